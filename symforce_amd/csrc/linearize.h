@@ -19,9 +19,10 @@ struct FactorGroup {
 // Linearizer::Relinearize (opt/linearizer.cc:57-112) on the device, without atomics. Pass 1, one
 // thread per factor and a launch per factor type: the residual into its rows and the factor's
 // local rhs J^T r and Hessian blocks J^T J (lower diagonal blocks, full off-diagonal blocks) into
-// a per-factor contribution record. Pass 2, one thread per rhs / hessian_lower entry: the sum of
-// its contributions, gathered through a host-built list in factor order (the order in which the
-// reference's UpdateFromLinearizedDenseFactorIntoSparse adds them, linearizer.cc:358-433).
+// a per-factor contribution record. Pass 2, per rhs / hessian_lower entry: the sum of its
+// contributions, gathered through a host-built list in factor order (the order in which the
+// reference's UpdateFromLinearizedDenseFactorIntoSparse adds them, linearizer.cc:358-433), by one
+// thread for a short list and by 16 lanes or a block with fixed strides for a long one.
 class CscLinearizer {
  public:
   void setup(const HostProblem& p, hipStream_t s);
@@ -33,7 +34,9 @@ class CscLinearizer {
  private:
   std::vector<FactorGroup> groups_;
   DBuf<double> contrib_;
-  DBuf<int32_t> hptr_, hidx_, rptr_, ridx_;  // gather lists: CSR over hval and rhs entries
+  DBuf<int32_t> ptr_, idx_;     // gather lists: CSR over the hval entries, then the rhs entries
+  DBuf<int32_t> group_, wide_;  // entries whose lists take 16 lanes / a block
+  int32_t n_group_ = 0, n_wide_ = 0;
 };
 
 }  // namespace symhip
