@@ -512,12 +512,33 @@ int symhip_cholesky_solve(symhip_cholesky_t c, const double* b, double* x, int32
   return guarded([&] {
     ensure_cholesky_device(c);
     const int32_t n = c->sym.n;
-    c->b.resize(std::max(1, n));
-    c->x.resize(std::max(1, n));
-    for (int32_t k = 0; k < nrhs; ++k) {
-      c->b.upload(b + (int64_t)k * n, n, c->stream);
-      c->ldlt.solve(c->b.get(), c->x.get(), c->stream);
-      c->x.download(x + (int64_t)k * n, n, c->stream);
+    // several right-hand sides go through the solver together, as many as its workspace takes
+    // (fewer, down to one at a time, where the device has no room for it)
+    int32_t per = nrhs > 1 && n > 0 ? c->ldlt.many_capacity(nrhs) : 1;
+    auto room = [&](int32_t m) {
+      const size_t need = (size_t)std::max(1, n) * m;
+      if (c->b.size() < need) c->b.resize(need);
+      if (c->x.size() < need) c->x.resize(need);
+      if (m > 1) c->ldlt.reserve_many(m, c->stream);
+    };
+    for (;;) {
+      try {
+        room(per);
+        break;
+      } catch (const symhip::Error&) {
+        if (per == 1) throw;
+        (void)hipGetLastError();
+        per /= 2;
+      }
+    }
+    for (int32_t k = 0; k < nrhs; k += per) {
+      const int32_t m = std::min(per, nrhs - k);
+      const size_t len = (size_t)n * m;
+      if (len) HIP_OK(hipMemcpyAsync(c->b.get(), b + (int64_t)k * n, len * sizeof(double),
+                                     hipMemcpyHostToDevice, c->stream));
+      if (per > 1) c->ldlt.solve_many(c->b.get(), c->x.get(), m, c->stream);
+      else c->ldlt.solve(c->b.get(), c->x.get(), c->stream);
+      c->x.download(x + (int64_t)k * n, len, c->stream);
     }
     HIP_OK(hipStreamSynchronize(c->stream));
   });

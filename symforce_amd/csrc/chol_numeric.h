@@ -26,6 +26,14 @@ class SupernodalLDLT {
   // x = A^-1 b for device vectors in the original (unpermuted) order; x may alias b.
   // Captured per (b, x) pair and replayed.
   void solve(const double* b, double* x, hipStream_t s);
+  // The same for nrhs right-hand sides stored one after the other (stride n), every level one launch
+  // for all of them; x may alias b. reserve_many allocates the workspace (three vectors per
+  // right-hand side, kept for later calls); many_capacity(nrhs) is how many to pass at a time so
+  // that it stays within kManyBytes together with the caller's own b and x.
+  void solve_many(const double* b, double* x, int32_t nrhs, hipStream_t s);
+  void reserve_many(int32_t nrhs, hipStream_t s);
+  int32_t many_capacity(int32_t nrhs) const;
+  static constexpr int64_t kManyBytes = 256 << 20;
   // x = A^-1 b for the b given to the last factorization (backward half only); x may alias b.
   void solve_fused(double* x, hipStream_t s);
   SupernodalLDLT() = default;
@@ -69,6 +77,8 @@ class SupernodalLDLT {
   CholSymbolic sym_;
   DBuf<double> panel_, l11_, D_, y_, yout_, part_;
   DBuf<int32_t> counter_;  // per-supernode arrival counters of the backward pass (self-resetting)
+  DBuf<double> many_y_, many_yout_, many_part_;  // solve_many
+  DBuf<int32_t> many_counter_;                   // per (right-hand-side group, supernode)
   DBuf<int64_t> asm_map_, scat_col_;
   DBuf<int32_t> rows_, perm_, upd_rel_, scat_rel_;
   DBuf<uint8_t> trsm_tasks_, upd_tasks_, solve_tasks_;  // per-level task lists (chol_numeric.hip)

@@ -656,6 +656,179 @@ __global__ void __launch_bounds__(256) bwd_kernel(const SnTask* __restrict__ tas
   }
 }
 
+// Several right-hand sides at once (covariances: every column of the identity). A block takes its
+// task's panel rows for a group of kRhsGroup right-hand sides (blockIdx.y), stored one after the
+// other with stride n: the panel and L11 are read once per group, each wavefront runs the
+// triangular solve of one of them, and a level is one launch whatever their number. One launch pair
+// per level per right-hand side left the chip to one block chain at a time: the 906 columns of a
+// 151-pose covariance took 202 ms from Hessian to dense inverse, now 4.0 (analysis and transfers
+// included).
+constexpr int kRhsGroup = 4;
+
+__global__ void __launch_bounds__(256) permute_many_kernel(int32_t n, int32_t nrhs,
+                                                           const int32_t* __restrict__ perm,
+                                                           const double* __restrict__ b,
+                                                           double* __restrict__ y,
+                                                           double* __restrict__ part) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  for (int32_t r = blockIdx.y; r < nrhs; r += gridDim.y) {
+    y[(int64_t)r * n + perm[i]] = b[(int64_t)r * n + i];
+    part[(int64_t)r * n + i] = 0.0;
+  }
+}
+__global__ void __launch_bounds__(256) unpermute_many_kernel(int32_t n, int32_t nrhs,
+                                                             const int32_t* __restrict__ perm,
+                                                             const double* __restrict__ y,
+                                                             double* __restrict__ x) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  for (int32_t r = blockIdx.y; r < nrhs; r += gridDim.y)
+    x[(int64_t)r * n + i] = y[(int64_t)r * n + perm[i]];
+}
+
+// Forward: as fwd_kernel; wave w solves right-hand side w of the group, then thread t takes below
+// row t % 128 for two of the four.
+__global__ void __launch_bounds__(256) fwd_many_kernel(const SnTask* __restrict__ tasks, int32_t n_all,
+                                                       int32_t nrhs,
+                                                       const int32_t* __restrict__ rows,
+                                                       const double* __restrict__ panel,
+                                                       const double* __restrict__ l11,
+                                                       double* __restrict__ yacc,
+                                                       double* __restrict__ yout) {
+  static_assert(kSolveRows == 128 && kRhsGroup == 4, "two halves of 128 threads, four wavefronts");
+  __shared__ double Ls[kMaxCols][kMaxCols + 1];
+  __shared__ double ys[kRhsGroup][kMaxCols];
+  const SnTask tk = tasks[blockIdx.x];
+  const int chunk = tk.a;
+  const SnDesc sd = tk.d;
+  const int n = sd.ncols, ld = sd.ld, mb = ld - n;
+  const double* P = panel + sd.panel_off;
+  const int32_t* rw = rows + sd.rows_off + n;
+  const int i = chunk * kSolveRows + (threadIdx.x & (kSolveRows - 1));
+  double lrow[kMaxCols];
+  {
+    const int64_t r = mb > 0 ? n + min(i, mb - 1) : 0;  // clamped into the panel
+#pragma unroll
+    for (int k = 0; k < kMaxCols; ++k) lrow[k] = P[(int64_t)min(k, n - 1) * ld + r];
+  }
+  stage_l11(l11 + sd.l11_off, n, Ls);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int rhs = blockIdx.y * kRhsGroup + wave;
+  double yi = 0;
+  if (rhs < nrhs && lane < n) yi = yacc[(int64_t)rhs * n_all + sd.col_begin + lane];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kMaxCols; ++k) yi -= Ls[lane][k] * lane_value(yi, k);
+  if (chunk == 0 && rhs < nrhs && lane < n) yout[(int64_t)rhs * n_all + sd.col_begin + lane] = yi;
+  ys[wave][lane] = lane < n ? yi : 0.0;
+  __syncthreads();
+  if (i < mb) {
+    const int32_t row = rw[i];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int g = 2 * (threadIdx.x / kSolveRows) + h, q = blockIdx.y * kRhsGroup + g;
+      if (q >= nrhs) break;
+      double acc = 0;
+#pragma unroll
+      for (int k = 0; k < kMaxCols; ++k) acc += lrow[k] * ys[g][k];
+      unsafeAtomicAdd(&yacc[(int64_t)q * n_all + row], -acc);
+    }
+  }
+}
+
+// Backward: as bwd_kernel (wave w forms the sums of columns w, w + 4, .. for the whole group); the
+// last chunk block of (s, group) solves the four right-hand sides, a wavefront each.
+__global__ void __launch_bounds__(256) bwd_many_kernel(const SnTask* __restrict__ tasks, int32_t n_all,
+                                                       int32_t n_snodes, int32_t nrhs,
+                                                       const int32_t* __restrict__ rows,
+                                                       const double* __restrict__ panel,
+                                                       const double* __restrict__ l11,
+                                                       const double* __restrict__ D,
+                                                       double* __restrict__ yout,
+                                                       double* __restrict__ part,
+                                                       int32_t* __restrict__ counter) {
+  constexpr int kPer = kMaxCols / 4;
+  __shared__ double Ls[kMaxCols][kMaxCols + 1];
+  __shared__ double red_all[4][kPer][64 + 1];
+  __shared__ int last;
+  const SnTask tk = tasks[blockIdx.x];
+  const int s = tk.s, chunk = tk.a;
+  const SnDesc sd = tk.d;
+  const int n = sd.ncols, ld = sd.ld, mb = ld - n;
+  const int nchunks = max(1, (mb + kSolveRows - 1) / kSolveRows);
+  const double* P = panel + sd.panel_off + n;
+  const int32_t* rw = rows + sd.rows_off + n;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  stage_l11(l11 + sd.l11_off, n, Ls);
+  const int rhs = blockIdx.y * kRhsGroup + wave;
+  double yown = 0;
+  if (rhs < nrhs && lane < n)
+    yown = yout[(int64_t)rhs * n_all + sd.col_begin + lane] / D[sd.col_begin + lane];
+  if (mb > 0) {
+    double acc[kRhsGroup][kPer] = {};
+#pragma unroll
+    for (int t = 0; t < kSolveRows / 64; ++t) {
+      const int i = chunk * kSolveRows + lane + 64 * t;
+      const int ic = min(i, mb - 1);
+      const int32_t row = rw[ic];
+      double yv[kRhsGroup];
+#pragma unroll
+      for (int g = 0; g < kRhsGroup; ++g) {
+        const int q = blockIdx.y * kRhsGroup + g;
+        const double yl = yout[(int64_t)min(q, nrhs - 1) * n_all + row];
+        yv[g] = (i < mb && q < nrhs) ? yl : 0.0;
+      }
+#pragma unroll
+      for (int c = 0; c < kPer; ++c) {
+        const double l = P[(int64_t)min(wave + 4 * c, n - 1) * ld + ic];
+#pragma unroll
+        for (int g = 0; g < kRhsGroup; ++g) acc[g][c] += l * yv[g];
+      }
+    }
+    auto red = red_all[wave];
+    const int c = lane >> 2, qtr = lane & 3, k = wave + 4 * c;
+#pragma unroll
+    for (int g = 0; g < kRhsGroup; ++g) {
+#pragma unroll
+      for (int e = 0; e < kPer; ++e) red[e][lane] = acc[g][e];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      double v = 0;
+#pragma unroll
+      for (int t = 0; t < 16; ++t) v += red[c][16 * qtr + t];
+      v += __shfl_xor(v, 1, 64);
+      v += __shfl_xor(v, 2, 64);
+      const int q = blockIdx.y * kRhsGroup + g;
+      if (qtr == 0 && k < n && q < nrhs)
+        unsafeAtomicAdd(&part[(int64_t)q * n_all + sd.col_begin + k], v);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();  // the next right-hand side overwrites red
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+  }
+  // every wave waits for its own atomics before the block arrives (as in bwd_kernel)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  int32_t* cnt = counter + (int64_t)blockIdx.y * n_snodes + s;
+  if (threadIdx.x == 0)
+    last = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+           nchunks - 1;
+  __syncthreads();
+  if (!__builtin_amdgcn_readfirstlane(last)) return;  // uniform across the block
+  if (threadIdx.x == 0) *cnt = 0;  // ready for the next solve
+  if (rhs >= nrhs) return;
+  double yi = 0;
+  if (lane < n)
+    yi = yown - (mb > 0 ? __hip_atomic_load(&part[(int64_t)rhs * n_all + sd.col_begin + lane],
+                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                        : 0.0);
+#pragma unroll
+  for (int k = kMaxCols - 1; k >= 0; --k) yi -= Ls[k][lane] * lane_value(yi, k);
+  if (lane < n) yout[(int64_t)rhs * n_all + sd.col_begin + lane] = yi;
+}
+
 }  // namespace
 
 void SupernodalLDLT::setup(const CholSymbolic& sym, const int32_t* colptr, const int32_t* rowind,
@@ -803,6 +976,52 @@ void SupernodalLDLT::factorize_assembled(hipStream_t s, const double* b) {
 void SupernodalLDLT::solve(const double* b, double* x, hipStream_t s) {
   if (sym_.n == 0) return;
   HIP_OK(hipGraphLaunch(cached_graph(solve_graphs_, b, x, s, [&] { launch_solve(b, x, s); }), s));
+}
+
+int32_t SupernodalLDLT::many_capacity(int32_t nrhs) const {
+  const int64_t per = 5 * sizeof(double) * (int64_t)std::max(1, sym_.n);  // y, yout, part, b, x
+  return (int32_t)std::min<int64_t>(nrhs, std::clamp<int64_t>(kManyBytes / per, kRhsGroup, 4096));
+}
+
+void SupernodalLDLT::reserve_many(int32_t nrhs, hipStream_t s) {
+  const size_t need = (size_t)sym_.n * nrhs;
+  const size_t cneed = (size_t)grid_for(nrhs, kRhsGroup) * sym_.n_snodes;
+  HIP_OK(hipStreamSynchronize(s));  // an earlier pass may still use the smaller buffers
+  for (auto* v : {&many_y_, &many_yout_, &many_part_})
+    if (v->size() < need) v->resize(need);
+  if (many_counter_.size() < cneed) {
+    many_counter_.resize(cneed);
+    fill_zero_i32(many_counter_.get(), (int64_t)cneed, s);
+  }
+}
+
+void SupernodalLDLT::solve_many(const double* b, double* x, int32_t nrhs, hipStream_t s) {
+  const int32_t n = sym_.n;
+  if (n == 0 || nrhs <= 0) return;
+  const int32_t groups = grid_for(nrhs, kRhsGroup);
+  SYMHIP_CHECK(many_part_.size() >= (size_t)n * nrhs &&
+                   many_counter_.size() >= (size_t)groups * sym_.n_snodes,
+               "internal: solve_many without reserve_many");
+  const SnTask* tasks = reinterpret_cast<const SnTask*>(solve_tasks_.get());
+  const dim3 pg(grid_for(n, 256), std::min(nrhs, 65535));
+  hipLaunchKernelGGL(permute_many_kernel, pg, dim3(256), 0, s, n, nrhs, perm_.get(), b,
+                     many_y_.get(), many_part_.get());
+  for (int l = 0; l < sym_.n_levels; ++l) {
+    const int nb = lvl_solve_ptr_[l + 1] - lvl_solve_ptr_[l];
+    hipLaunchKernelGGL(fwd_many_kernel, dim3(nb, groups), dim3(256), 0, s,
+                       tasks + lvl_solve_ptr_[l], n, nrhs, rows_.get(), panel_.get(), l11_.get(),
+                       many_y_.get(), many_yout_.get());
+  }
+  for (int l = sym_.n_levels - 1; l >= 0; --l) {
+    const int nb = lvl_solve_ptr_[l + 1] - lvl_solve_ptr_[l];
+    hipLaunchKernelGGL(bwd_many_kernel, dim3(nb, groups), dim3(256), 0, s,
+                       tasks + lvl_solve_ptr_[l], n, sym_.n_snodes, nrhs, rows_.get(),
+                       panel_.get(), l11_.get(), D_.get(), many_yout_.get(), many_part_.get(),
+                       many_counter_.get());
+  }
+  hipLaunchKernelGGL(unpermute_many_kernel, pg, dim3(256), 0, s, n, nrhs, perm_.get(),
+                     many_yout_.get(), x);
+  HIP_OK(hipGetLastError());
 }
 
 void SupernodalLDLT::solve_fused(double* x, hipStream_t s) {
