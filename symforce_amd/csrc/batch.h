@@ -61,7 +61,7 @@ class BatchLocalization {
   int64_t storage_total() const { return (int64_t)cvals_host_size_; }
 
  private:
-  int32_t n_problems_ = 0, total_poses_ = 0;
+  int32_t n_problems_ = 0, total_poses_ = 0, max_poses_ = 0;
   symhip_optimizer_params p_;
   bool f32_ = false;
   double eps_ = 0;

@@ -7,8 +7,10 @@
 // consecutive poses and matching factors touch one pose, so H is block tridiagonal with 6 x 6
 // blocks. Lane i linearizes pose i (its matching factors and the odometry factor to pose i + 1,
 // whose pose-(i + 1) terms are handed to lane i + 1 by a shuffle); the wavefront then solves the
-// damped system by block-tridiagonal Cholesky, six lanes holding the rows of each 6 x 6 block. Per state block and pose the linearization keeps
-// 63 doubles: the lower diagonal block (21), H(i + 1, i) (36, row-major) and the rhs (6).
+// damped system by a block-tridiagonal LDL^T from both ends of the chain at once. Per state block
+// and pose the linearization keeps 63 doubles: the lower diagonal block (21), H(i + 1, i) (36,
+// row-major) and the rhs (6), entry by entry over the poses so that a wavefront's lanes read and
+// write consecutive addresses.
 #include "./batch.h"
 
 #include <algorithm>
@@ -16,6 +18,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "./dpp.h"
 #include "./factor_traits.h"
 #include "./geo.h"
 #include "./lm_logic.h"
@@ -27,6 +30,9 @@ namespace symhip {
 namespace {
 
 constexpr int kLin = 63;
+// offsets of a pose's record: lower diagonal block, H(i + 1, i), rhs
+constexpr int kRecB = 21, kRecX = 57;
+constexpr int kRec = 65;  // LDS stride of a pose's record (odd: lanes on their own poses spread over the banks)
 constexpr int kMaxPoses = 64;
 
 struct BatchView {
@@ -38,7 +44,7 @@ struct BatchView {
   const int32_t* odo_args;    // 3 per pose: measurement, sigmas, epsilon offsets (-1: last pose)
   const double* cvals;
   double* vals;  // [3][total_poses][7]
-  double* lin;   // [3][total_poses][kLin]
+  double* lin;   // [3][kLin][total_poses]
   double* maxd;  // [total_poses][6]
   double* vout;  // storage copy; best poses written back
   symhip_iteration_stats* recs;
@@ -49,8 +55,9 @@ struct BatchView {
 };
 
 __device__ __forceinline__ double wave_total(double v) {
+  v = xor16_sum(xor32_sum(v));
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
 
@@ -65,39 +72,17 @@ __device__ __forceinline__ int tri(int r, int c) { return r * (r + 1) / 2 + c; }
 // in FP64 from the FP32 Jacobians, so H stays positive semi-definite (FP32 sums of products
 // made a near-singular H slightly indefinite, and the block Cholesky then failed).
 template <typename S>
-__device__ double linearize(const BatchView& v, int b, int64_t g, int lane, bool live) {
-  double D[21] = {}, gv[6] = {}, Bv[36] = {}, Dn[21] = {}, gn[6] = {};
+__device__ __forceinline__ double linearize(const BatchView& v, int b, int g0, int n, int lane) {
+  double D[21] = {}, gv[6] = {}, Dn[21] = {}, gn[6] = {};
   double e = 0;
   int has_next = 0;
+  const bool live = lane < n;
+  const int g = g0 + min(lane, n - 1);
+  const int64_t TP = v.total_poses;
+  double* lin = v.lin + (int64_t)b * kLin * TP;  // entry k of pose g at lin[k * TP + g]
+  auto put = [&](int k, double x) { (lin + k * TP)[g] = x; };
   if (live) {
-    const double* pose = v.vals + (b * v.total_poses + g) * 7;
-    for (int m = v.match_ptr[g]; m < v.match_ptr[g + 1]; ++m) {
-      const double* a[4] = {pose, v.cvals + v.match_args[3 * m], v.cvals + v.match_args[3 * m + 1],
-                            v.cvals + v.match_args[3 * m + 2]};
-      S rs[3], J[3][6];
-      factor_matching<S>(a, rs, J);
-      double r[3], Jd[3][6];
-      if constexpr (std::is_same_v<S, double>) {
-#pragma unroll
-        for (int q = 0; q < 3; ++q) r[q] = rs[q];
-      } else {
-        factor_matching<double>(a, r, Jd);
-      }
-#pragma unroll
-      for (int i = 0; i < 6; ++i) {
-#pragma unroll
-        for (int q = 0; q < 3; ++q) gv[i] += (double)J[q][i] * r[q];
-#pragma unroll
-        for (int j = 0; j <= i; ++j) {
-          double h = 0;
-#pragma unroll
-          for (int q = 0; q < 3; ++q) h += (double)J[q][i] * (double)J[q][j];
-          D[tri(i, j)] += h;
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < 3; ++q) e += r[q] * r[q];
-    }
+    const double* pose = v.vals + (b * TP + g) * 7;
     const int32_t* oa = v.odo_args + 3 * g;
     if (oa[0] >= 0) {
       has_next = 1;
@@ -111,37 +96,38 @@ __device__ double linearize(const BatchView& v, int b, int64_t g, int lane, bool
       } else {
         factor_odometry<double>(a, r, Jd);
       }
+      // sum_q J[q][i] J[q][j] over the residual rows where both columns have entries: rotation
+      // columns of the first pose touch all six rows, those of the second the first three,
+      // translation columns the last three (factor_odometry); the other products are zeros.
+      auto dot = [&](int i, int j, int q0, int q1) {
+        double h = 0;
+        for (int q = q0; q < q1; ++q) h += (double)J[q][i] * (double)J[q][j];
+        return h;
+      };
 #pragma unroll
       for (int i = 0; i < 6; ++i) {
         double ga = 0, gb = 0;
-#pragma unroll
-        for (int q = 0; q < 6; ++q) {
-          ga += (double)J[q][i] * r[q];
-          gb += (double)J[q][6 + i] * r[q];
-        }
-        gv[i] += ga;
+        for (int q = i < 3 ? 0 : 3; q < 6; ++q) ga += (double)J[q][i] * r[q];
+        for (int q = i < 3 ? 0 : 3; q < (i < 3 ? 3 : 6); ++q) gb += (double)J[q][6 + i] * r[q];
+        gv[i] = ga;
         gn[i] = gb;
+        // H(i + 1, i), rows of the next pose, columns of this one: stored as it is formed
 #pragma unroll
         for (int j = 0; j < 6; ++j) {
-          double hb = 0;
-#pragma unroll
-          for (int q = 0; q < 6; ++q) hb += (double)J[q][6 + i] * (double)J[q][j];
-          Bv[i * 6 + j] = hb;  // H(i + 1, i): rows of pose i + 1, cols of pose i
+          const double hb = i < 3 ? (j < 3 ? dot(6 + i, j, 0, 3) : 0.0) : dot(6 + i, j, 3, 6);
+          put(kRecB + i * 6 + j, hb);
         }
 #pragma unroll
         for (int j = 0; j <= i; ++j) {
-          double ha = 0, hn = 0;
-#pragma unroll
-          for (int q = 0; q < 6; ++q) {
-            ha += (double)J[q][i] * (double)J[q][j];
-            hn += (double)J[q][6 + i] * (double)J[q][6 + j];
-          }
-          D[tri(i, j)] += ha;
-          Dn[tri(i, j)] = hn;
+          D[tri(i, j)] = j < 3 && i < 3 ? dot(i, j, 0, 6) : dot(i, j, 3, 6);
+          Dn[tri(i, j)] = i < 3 ? dot(6 + i, 6 + j, 0, 3) : (j < 3 ? 0.0 : dot(6 + i, 6 + j, 3, 6));
         }
       }
 #pragma unroll
       for (int q = 0; q < 6; ++q) e += r[q] * r[q];
+    } else {
+#pragma unroll
+      for (int k = 0; k < 36; ++k) put(kRecB + k, 0.0);
     }
   }
   // the odometry factor's pose-(i + 1) terms belong to the next lane
@@ -157,23 +143,87 @@ __device__ double linearize(const BatchView& v, int b, int64_t g, int lane, bool
     const double t = __shfl_up(gn[k], 1, 64);
     if (take) gv[k] += t;
   }
+  // The matching factors. A problem of at most 32 (16) poses gives each pose two (four) lanes,
+  // lane + 32 (lane + 16, ..), which take its factors in turn. A lane takes kMatch of them at a
+  // time: their offsets in one round of loads, their inputs in the next (one factor after the
+  // other waits for both rounds; the compiler sinks a hand-pipelined loop's loads back to their
+  // uses). Past the list's end the last factor repeats with an infinite sigma, which adds zeros.
+  {
+    constexpr int kMatch = 4;
+    const int stride = n <= 16 ? 16 : n <= 32 ? 32 : 64;
+    const int parts = 64 / stride, i = lane & (stride - 1), part = lane / stride;
+    const int gm = g0 + min(i, n - 1);
+    const double* pose = v.vals + (b * TP + gm) * 7;
+    const int m0 = v.match_ptr[gm], m1 = i < n ? v.match_ptr[gm + 1] : m0;
+    double p[7];
+#pragma unroll
+    for (int k = 0; k < 7; ++k) p[k] = pose[k];
+    for (int m = m0 + part; m < m1; m += kMatch * parts) {
+      int32_t o[kMatch][3];
+#pragma unroll
+      for (int t = 0; t < kMatch; ++t)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) o[t][k] = v.match_args[3 * min(m + t * parts, m1 - 1) + k];
+      double lm[kMatch][3], meas[kMatch][3], sigma[kMatch];
+#pragma unroll
+      for (int t = 0; t < kMatch; ++t) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          lm[t][k] = v.cvals[o[t][0] + k];
+          meas[t][k] = v.cvals[o[t][1] + k];
+        }
+        sigma[t] = v.cvals[o[t][2]];
+      }
+#pragma unroll
+      for (int t = 0; t < kMatch; ++t) {
+        const double sg = m + t * parts < m1 ? sigma[t] : __builtin_huge_val();
+        const double* a[4] = {p, lm[t], meas[t], &sg};
+        S rs[3], J[3][6];
+        factor_matching<S>(a, rs, J);
+        double r[3], Jd[3][6];
+        if constexpr (std::is_same_v<S, double>) {
+#pragma unroll
+          for (int q = 0; q < 3; ++q) r[q] = rs[q];
+        } else {
+          factor_matching<double>(a, r, Jd);
+        }
+        // rotation column c has no entry in row c (a cross product's matrix)
+#pragma unroll
+        for (int c = 0; c < 6; ++c)
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            if (q == c) continue;
+            const double jc = (double)J[q][c];
+            gv[c] = fma(jc, r[q], gv[c]);
+#pragma unroll
+            for (int d = 0; d <= c; ++d)
+              if (q != d) D[tri(c, d)] = fma(jc, (double)J[q][d], D[tri(c, d)]);
+          }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) e = fma(r[q], r[q], e);
+      }
+    }
+    // the lanes of a pose together
+    if (parts > 1) {
+#pragma unroll
+      for (int k = 0; k < 21; ++k) D[k] = xor32_sum(D[k]);
+#pragma unroll
+      for (int k = 0; k < 6; ++k) gv[k] = xor32_sum(gv[k]);
+    }
+    if (parts > 2) {
+#pragma unroll
+      for (int k = 0; k < 21; ++k) D[k] = xor16_sum(D[k]);
+#pragma unroll
+      for (int k = 0; k < 6; ++k) gv[k] = xor16_sum(gv[k]);
+    }
+  }
   if (live) {
-    double* L = v.lin + (b * v.total_poses + g) * kLin;
 #pragma unroll
-    for (int k = 0; k < 21; ++k) L[k] = D[k];
+    for (int k = 0; k < 21; ++k) put(k, D[k]);
 #pragma unroll
-    for (int k = 0; k < 36; ++k) L[21 + k] = Bv[k];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) L[57 + k] = gv[k];
+    for (int k = 0; k < 6; ++k) put(kRecX + k, gv[k]);
   }
   return 0.5 * wave_total(e);
-}
-
-// Value of v in lane k (k wave-uniform) through two scalar lane reads.
-__device__ __forceinline__ double lane_bcast(double v, int k) {
-  const int2 u = __builtin_bit_cast(int2, v);
-  return __builtin_bit_cast(double, make_int2(__builtin_amdgcn_readlane(u.x, k),
-                                              __builtin_amdgcn_readlane(u.y, k)));
 }
 
 __device__ __forceinline__ void wave_lds_sync() {
@@ -182,187 +232,240 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Block-tridiagonal Cholesky H = L L^T (L block lower bidiagonal: C_i on the diagonal,
-// W_i = B_i C_i^-T below) and the two triangular solves, by the whole wavefront: lane r < 6
-// holds row r of the 6 x 6 blocks of the current pose (the other lanes shadow row 5), and the
-// values another row needs cross by scalar lane reads, so a pose costs a few dozen dependent
-// steps instead of the ~6 000 cycles of one lane doing every entry. Each entry is formed by the
-// same operations in the same order as a one-lane sweep would form it. A: packed lower diagonal
-// blocks (overwritten by C_i), B: H(i + 1, i) row-major (overwritten by W_i), x: rhs in,
-// H^-1 rhs out (LDS, written by the row lanes, read back after a wavefront fence).
-__device__ void block_tridiagonal_solve(int n, double (*A)[21], double (*B)[36], double (*x)[6],
-                                        int lane) {
-  const int r = lane < 6 ? lane : 5;
-  const bool row = lane < 6;
-  double wprev[6] = {}, yprev[6] = {};
-  for (int i = 0; i < n; ++i) {
-    // M = A_i - W_{i-1} W_{i-1}^T, row r (entries c <= r)
-    double m[6];
+// Block-tridiagonal LDL^T of H and the two triangular solves, by the whole wavefront, from both
+// ends of the chain towards its middle pose m = n / 2 (no fill: each half's elimination touches its
+// own poses only, and the middle block takes an update from either side). The row of lanes 0..15
+// eliminates poses 0, 1, .. m - 1, the row of lanes 16..31 poses n - 1, n - 2, .. m + 1 (one fewer
+// when n is even: its first step is an identity pose), the upper two rows repeat them.
+//
+// Inside a row, a step's lanes hold the rows of [A_i; B; x_i^T]: six pivot rows of the pose's
+// diagonal block, the six rows that its coupling block gives the next pose towards the middle, and
+// the right-hand side as a thirteenth row. All of them undergo the same elimination: for column k,
+// d = pivot k, l = own entry / d, and the columns after it lose l times the pivot rows' entries,
+// which cross the row of lanes by row_bcast. Each non-pivot row then forms its row of the next
+// pose's update, -sum_k l_k w_ck (w = l d, row c's from its lane), so the next diagonal block and
+// right-hand side appear in the lanes that held the coupling block: pivot rows alternate between
+// lanes 0..5 and 6..11 from step to step, and nothing moves. In the records (LDS) A's strict lower
+// part is overwritten by -L, B by the coupling rows' -l, x by -D^-1 L^-1 x and then by the solution.
+//
+// A step's dependent chain is six reciprocals with their updates, ~0.3 us: one row of lanes
+// eliminating the whole chain by Cholesky, with scalar lane reads, square roots and divisions, took
+// four times as long per pose and twice the poses (4096 problems of 5-50 poses: 1.98 ms a launch,
+// one wavefront per SIMD; with this and the linearization above 0.43).
+//
+// Columns K.. of a step whose pivot rows are in lanes kBase.. of each row of lanes and whose coupling
+// rows are in lanes kCouple..: v's column K becomes the unscaled w_K, nl_K = -w_K / d_K, and acc_c
+// collects sum_k nl_k w_ck with w_ck from lane kCouple + c (each column's share as soon as its nl
+// is there, behind the next column's reciprocal).
+template <int kBase, int kCouple, int K = 0>
+__device__ __forceinline__ void eliminate(double (&v)[6], double (&nl)[6], double (&acc)[6]) {
+  if constexpr (K < 6) {
+    const double w = v[K];
+    nl[K] = w * -refined_rcp(row_bcast<kBase + K>(w));
+    row_fmac<kBase + K + 1, 5 - K>(v + K + 1, w, nl[K]);
+    row_fmac<kCouple, 6>(acc, w, nl[K]);
+    eliminate<kBase, kCouple, K + 1>(v, nl, acc);
+  }
+}
+// t_c += nl(q, c) x_q for q = 5 .. 1, x_q = t of lane q (lc[q] = nl(q, own c), zero where c >= q)
+template <int Q = 5>
+__device__ __forceinline__ void back_columns(double& t, const double (&lc)[6]) {
+  if constexpr (Q > 0) {
+    t = fma(lc[Q], row_bcast<Q>(t), t);
+    back_columns<Q - 1>(t, lc);
+  }
+}
+// t += sum_r wc_r x_r, x_r from lane r (wc_r = nl of coupling row r, own column)
+template <int R = 0>
+__device__ __forceinline__ void back_coupling(double& t, const double (&wc)[6], double x) {
+  if constexpr (R < 6) {
+    t = fma(wc[R], row_bcast<R>(x), t);
+    back_coupling<R + 1>(t, wc, x);
+  }
+}
+
+__device__ __forceinline__ void block_tridiagonal_solve(int n, double* rec, int lane) {
+  const int q = lane & 15;
+  const bool second = (lane >> 4) & 1;  // the chain from the far end
+  const int m = n >> 1;                    // the middle pose: m steps on the first chain,
+  const int skip = m - (n - 1 - m);        // m - skip on the second
+  // offsets of this lane's row in a pose's record, as a pivot row, a coupling row (row r of the
+  // pose towards the middle; the second chain's block is stored transposed) or the rhs row, for the
+  // two alternating lane roles; kept as row r and its role
+  const int r0 = q < 6 ? q : q - 6;
+  auto offset = [&](bool pivot, bool rhs, int c) {
+    const int a = c <= r0 ? tri(r0, c) : tri(c, r0);
+    const int b = kRecB + (second ? c * 6 + r0 : r0 * 6 + c);
+    return rhs ? kRecX + c : pivot ? a : b;
+  };
+  const bool rhs_row = q >= 12;
+  // the pose of step s on this lane's chain (clamped at the second chain's identity step)
+  auto pose_of = [&](int s) { return second ? min(n - 1, n - 1 - (s - skip)) : s; };
+  auto is_pivot = [&](int par) { return par == 0 ? q < 6 : q >= 6 && !rhs_row; };
+  // a coupling row of the second chain is in the record of the pose before its own
+  auto record = [&](int s, int par) {
+    const int p = pose_of(s);
+    return (!is_pivot(par) && !rhs_row && second ? max(p - 1, 0) : p) * kRec;
+  };
+  // Rows are read whole and written but for a pivot row's entries from its diagonal on: those go
+  // to the record's padding, and all entries of lanes that have nothing to store (the repeating
+  // rows of lanes, the spare lanes, the identity pose) to the spare record, without a branch.
+  int off[2][6], put[2][6];
 #pragma unroll
-    for (int c = 0; c < 6; ++c) m[c] = A[i][tri(r, c <= r ? c : r)];
-    if (i > 0) {
+  for (int par = 0; par < 2; ++par)
 #pragma unroll
-      for (int c = 0; c < 6; ++c) {
-        double sum = 0;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) sum += wprev[k] * B[i - 1][c * 6 + k];
-        m[c] -= sum;
-      }
+    for (int c = 0; c < 6; ++c) {
+      off[par][c] = offset(is_pivot(par), rhs_row, c);
+      put[par][c] = is_pivot(par) && c >= r0 ? kLin : off[par][c];
     }
-    // Cholesky of M; every entry of C_i ends up in Cb (uniform) on the way
-    // (one reciprocal per column; the triangular solves below multiply by it)
-    double Cb[6][6], Ci[6];
+  const bool writer = lane < 32 && q <= 12;
+  double acc[6] = {}, cur[6], nl[6];
+  auto load = [&](int s, int par) {
+    const double* x = rec + record(s, par);
 #pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      const double ckk = sqrt(lane_bcast(m[k], k));
-      Cb[k][k] = ckk;
-      Ci[k] = 1.0 / ckk;
-      const double lrk = m[k] * Ci[k];  // row r's entry of column k (r > k)
+    for (int c = 0; c < 6; ++c) cur[c] = x[off[par][c]];
+  };
+  auto step = [&]<int kPar>(int s) __attribute__((always_inline)) {
+    constexpr int kPivot = kPar ? 6 : 0, kCouple = kPar ? 0 : 6;
+    double v[6];
 #pragma unroll
-      for (int c = k + 1; c < 6; ++c) Cb[c][k] = lane_bcast(lrk, c);
-      if (r > k) m[k] = lrk;
-      else if (r == k) m[k] = ckk;
+    for (int c = 0; c < 6; ++c) v[c] = cur[c] + acc[c];
+    load(min(s + 1, m - 1), kPar ^ 1);  // the next step's rows (not used after the last one)
 #pragma unroll
-      for (int c = k + 1; c < 6; ++c)
-        if (c <= r && r > k) m[c] -= lrk * Cb[c][k];
+    for (int c = 0; c < 6; ++c) acc[c] = 0.0;
+    eliminate<kPivot, kCouple>(v, nl, acc);
+    double* x = rec + (writer && !(second && s < skip) ? record(s, kPar) : n * kRec);
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+      x[put[kPar][c]] = nl[c];
+      acc[c] = is_pivot(kPar) ? 0.0 : acc[c];  // these lanes take coupling rows next
     }
-    if (row) {
+  };
+  if (m > 0) {
+    load(0, 0);
+    if (second && skip > 0) {  // the identity pose: nothing couples
 #pragma unroll
-      for (int c = 0; c < 6; ++c)
-        if (c <= r) A[i][tri(r, c)] = m[c];
+      for (int c = 0; c < 6; ++c) cur[c] = q < 6 && c == r0 ? 1.0 : 0.0;
     }
-    // W_i row r = B_i row r C_i^-T, and y_i = C_i^-1 (x_i - W_{i-1} y_{i-1})
-    double w[6];
-    if (i + 1 < n) {
-#pragma unroll
-      for (int c = 0; c < 6; ++c) {
-        double v = B[i][r * 6 + c];
-#pragma unroll
-        for (int k = 0; k < c; ++k) v -= w[k] * Cb[c][k];
-        w[c] = v * Ci[c];
-      }
-    }
-    double b = x[i][r];
-    if (i > 0) {
-#pragma unroll
-      for (int k = 0; k < 6; ++k) b -= wprev[k] * yprev[k];
-    }
-    double bu[6], y[6];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) bu[k] = lane_bcast(b, k);
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-      double v = bu[q];
-#pragma unroll
-      for (int k = 0; k < q; ++k) v -= Cb[q][k] * y[k];
-      y[q] = v * Ci[q];
-    }
-    if (row) {
-      x[i][r] = y[r < 6 ? r : 5];
-      if (i + 1 < n) {
-#pragma unroll
-        for (int c = 0; c < 6; ++c) B[i][r * 6 + c] = w[c];
-      }
-    }
-    wave_lds_sync();  // W_i is read by all rows at pose i + 1
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      wprev[k] = w[k];
-      yprev[k] = y[k];
+    for (int s = 0; s < m; s += 2) {
+      step.template operator()<0>(s);
+      if (s + 1 < m) step.template operator()<1>(s + 1);
     }
   }
-  // x_i = C_i^-T (y_i - W_i^T x_{i+1})
-  double xnext[6] = {};
-  for (int i = n - 1; i >= 0; --i) {
-    double b = x[i][r];
-    if (i + 1 < n) {
+  // The middle pose: its own block and right-hand side, plus the update of either chain.
+  auto middle = [&]<int kPar>() __attribute__((always_inline)) {
+    constexpr int kPivot = kPar ? 6 : 0;
+    const bool row = is_pivot(kPar) || rhs_row;
+    double v[6];
 #pragma unroll
-      for (int k = 0; k < 6; ++k) b -= B[i][k * 6 + r] * xnext[k];
+    for (int c = 0; c < 6; ++c) {
+      const double x = rec[m * kRec + off[kPar][c]];
+      const double mine = acc[c] + (second ? 0.0 : x);
+      const double both = xor16_sum(mine);
+      v[c] = row ? both : 0.0;
     }
-    double bu[6], xs[6], di[6];
+    double unused[6] = {};
+    eliminate<kPivot, 0>(v, nl, unused);
+    double* x = rec + (lane < 13 && row ? m : n) * kRec;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) x[put[kPar][c]] = nl[c];
+  };
+  if (m & 1) middle.template operator()<1>(); else middle.template operator()<0>();
+  wave_lds_sync();  // the factor's rows are read by columns below
+  // Back from the middle: x_i = L^-T (D^-1 L^-1 x_i - W^T x_next), lane c of a row holding column c.
+  const int c = min(q, 5);
+  int lo[6], wo[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    lo[k] = tri(k, c < k ? c : 0);
+    wo[k] = kRecB + (second ? c * 6 + k : k * 6 + c);
+  }
+  double x = 0, lc[6], wc[6], z = 0;
+  auto load_back = [&](int s) {
+    const int p = s == m ? m : pose_of(s);
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
-      bu[k] = lane_bcast(b, k);
-      di[k] = 1.0 / A[i][tri(k, k)];  // off the substitution's dependent chain
+      const double t = rec[p * kRec + lo[k]];
+      lc[k] = c < k ? t : 0.0;
+      wc[k] = s == m ? 0.0 : rec[(second ? max(p - 1, 0) : p) * kRec + wo[k]];
     }
+    z = rec[p * kRec + kRecX + c];
+  };
+  load_back(m);
+  for (int s = m; s >= 0; --s) {
+    double t = -z;
+    back_coupling(t, wc, x);
+    double lq[6];
 #pragma unroll
-    for (int q = 5; q >= 0; --q) {
-      double v = bu[q];
-#pragma unroll
-      for (int k = q + 1; k < 6; ++k) v -= A[i][tri(k, q)] * xs[k];
-      xs[q] = v * di[q];
-    }
-    if (row) x[i][r] = xs[r < 6 ? r : 5];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) xnext[k] = xs[k];
+    for (int k = 0; k < 6; ++k) lq[k] = lc[k];
+    if (s > 0) load_back(s - 1);
+    back_columns(t, lq);
+    x = t;
+    const int p = s == m ? m : pose_of(s);
+    if (q < 6 && (s == m ? lane < 16 : lane < 32 && !(second && s < skip)))
+      rec[p * kRec + kRecX + c] = x;
   }
   wave_lds_sync();
 }
 
-// kWaves: wavefronts per SIMD the register allocation must allow (1: no spills, the linearization
-// holds ~350 VGPRs; 2: twice the resident problems at the cost of ~120 spilled registers); the
-// batch autotuner picks per batch.
+// LDS of a launch whose largest problem has max_poses poses (the launches that do not know it take
+// kMaxPoses: four problems per CU; 50 poses: six).
+constexpr uint32_t rec_bytes(int32_t max_poses) {
+  return (uint32_t)((max_poses + 1) * kRec * sizeof(double));
+}
+
+// kWaves: wavefronts per SIMD the register allocation must allow (1: no spills, ~360 VGPRs; 2: as
+// many more resident problems as their LDS records leave room for, at the cost of spilled
+// registers); the batch autotuner picks per batch.
 template <typename S, int kWaves>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWaves)))
 batch_lm_kernel(BatchView v, symhip_optimizer_params p, double eps) {
-  __shared__ double sA[kMaxPoses][21];
-  __shared__ double sB[kMaxPoses][36];
-  __shared__ double sx[kMaxPoses][6];
+  extern __shared__ double rec[];  // a record per pose and a spare one (rec_bytes)
   const int prob = v.order ? v.order[blockIdx.x] : (int)blockIdx.x, lane = threadIdx.x;
   const int64_t t_start = wall_clock64();
   const int g0 = v.pose_begin[prob], n = v.pose_begin[prob + 1] - g0;
   const bool live = lane < n;
-  const int64_t g = g0 + min(lane, n - 1);
+  const int g = g0 + min(lane, n - 1);
   const int64_t TP = v.total_poses;
   // Reset: the start Values go into the New block (block 1)
-  if (live)
-    for (int k = 0; k < 7; ++k) v.vals[(TP + g) * 7 + k] = v.cvals[v.pose_soff[g] + k];
+  if (live) {
+    const double* src = v.cvals + v.pose_soff[g];
+    double t[7];
+    for (int k = 0; k < 7; ++k) t[k] = src[k];
+    for (int k = 0; k < 7; ++k) v.vals[(TP + g) * 7 + k] = t[k];
+  }
   // the first linearization reads the next lane's start pose (odometry), written just above
   __syncthreads();
-  int init = 0, nw = 1, best = 0, fre = 2, iteration = -1, best_index = 0;
-  int status = 0, reason = 0, linearized = 0, nrec = 0;
+  // the state blocks as Iterate's first step and first linearization leave them
+  int init = 1, nw = 0, best = 1, fre = 2, best_index = 0;
+  int status = 0, reason = 0, nrec = 0;
   bool have_max = false, done = false;
   double err[3] = {0, 0, 0};
   double lambda = p.initial_lambda, nu = p.dynamic_lambda_update_beta;
-  auto record = [&](const symhip_iteration_stats& r) {
+  auto record = [&](const symhip_iteration_stats& r) __attribute__((always_inline)) {
     if (lane == 0 && v.recs && nrec < v.rec_stride)
       v.recs[(int64_t)prob * v.rec_stride + nrec] = r;
     ++nrec;
   };
-  auto relin = [&](int b) {
-    err[b] = linearize<S>(v, b, g, lane, live);
-    linearized |= 1 << b;
-  };
-  for (int it = 0; it < p.iterations && !done; ++it) {
-    const int t = init;
-    init = nw;
-    nw = t;
-    ++iteration;
-    if (!((linearized >> init) & 1)) {
-      relin(init);
-      if (best != init) {
-        if (best != nw) fre = best;
-        best = init;
-      }
-    }
-    if (iteration == 0) {
-      symhip_iteration_stats r{};
-      r.iteration = -1;
-      r.new_error = err[init];
-      r.current_lambda = lambda;
-      record(r);
-      if (!isfinite(err[init])) {
-        status = SYMHIP_STATUS_FAILED;
-        reason = SYMHIP_FAILURE_INITIAL_ERROR_NOT_FINITE;
-        break;
-      }
-    }
+  // One damped step: New = Init retracted by the update. Returns this lane's share of the linear
+  // error's update . (rhs - damping * update).
+  auto take_step = [&]() __attribute__((always_inline)) {
+    double lde = 0;
     // DampHessian (levenberg_marquardt_solver.tcc:22-54) out of place, and the staged system
-    const double* Li = v.lin + (init * TP + g) * kLin;
-    double damp[6] = {}, u[6] = {};
+    const double* lin = v.lin + (int64_t)init * kLin * TP;  // entry k of pose g at lin[k * TP + g]
+    double damp[6] = {}, u[6] = {}, rhs[6] = {};
     if (live) {
+      double* own = rec + lane * kRec;
+      double t[kLin];
+#pragma unroll
+      for (int k = 0; k < kLin; ++k) t[k] = (lin + k * TP)[g];
+      __builtin_amdgcn_sched_barrier(0);  // all loads in flight before the first LDS write
+#pragma unroll
+      for (int k = 0; k < kLin; ++k) own[k] = t[k];
+#pragma unroll
       for (int k = 0; k < 6; ++k) {
-        const double dk = Li[tri(k, k)];
+        rhs[k] = t[kRecX + k];
+        const double dk = t[tri(k, k)];
         double d = 0;
         if (p.use_diagonal_damping) {
           if (p.keep_max_diagonal_damping) {
@@ -375,21 +478,18 @@ batch_lm_kernel(BatchView v, symhip_optimizer_params p, double eps) {
         }
         if (p.use_unit_damping) d += lambda;
         damp[k] = d;
+        own[tri(k, k)] = dk + d;
       }
-      for (int k = 0; k < 21; ++k) sA[lane][k] = Li[k];
-      for (int k = 0; k < 6; ++k) sA[lane][tri(k, k)] += damp[k];
-      for (int k = 0; k < 36; ++k) sB[lane][k] = Li[21 + k];
-      for (int k = 0; k < 6; ++k) sx[lane][k] = Li[57 + k];
     }
     if (p.use_diagonal_damping && p.keep_max_diagonal_damping) have_max = true;
     __syncthreads();
-    block_tridiagonal_solve(n, sA, sB, sx, lane);
+    block_tridiagonal_solve(n, rec, lane);
     __syncthreads();
-    double lde = 0;
     if (live) {
+#pragma unroll
       for (int k = 0; k < 6; ++k) {
-        u[k] = -sx[lane][k];
-        lde += u[k] * (Li[57 + k] - damp[k] * u[k]);
+        u[k] = -rec[lane * kRec + kRecX + k];
+        lde += u[k] * (rhs[k] - damp[k] * u[k]);
       }
       // UpdateNewFromInit: New = Init retracted by the update
       const double* src = v.vals + (init * TP + g) * 7;
@@ -400,20 +500,55 @@ batch_lm_kernel(BatchView v, symhip_optimizer_params p, double eps) {
       dst[5] += u[4];
       dst[6] += u[5];
     }
-    __syncthreads();  // sA/sB/sx are rewritten next iteration
-    relin(nw);
+    __syncthreads();  // the records are rewritten next iteration
+    return lde;
+  };
+  // One body for the start's linearization (iteration -1, of Init) and each step's (of New): the
+  // code is fetched as it runs, a few times per launch, and a second copy of the linearization
+  // costs more than the branches.
+  int iteration = -1;
+  while (iteration < p.iterations && !done) {
+    double lde = 0;
+    if (iteration >= 1) {
+      const int t = init;
+      init = nw;
+      nw = t;
+    }
+    if (iteration >= 0) lde = take_step();
+    const double e_new = linearize<S>(v, iteration < 0 ? init : nw, g0, n, lane);
+    if (iteration < 0) {
+      err[init] = e_new;
+      symhip_iteration_stats r{};
+      r.iteration = -1;
+      r.new_error = e_new;
+      r.current_lambda = lambda;
+      record(r);
+      if (!isfinite(e_new)) {
+        status = SYMHIP_STATUS_FAILED;
+        reason = SYMHIP_FAILURE_INITIAL_ERROR_NOT_FINITE;
+        break;
+      }
+      iteration = 0;
+      asm volatile("" : "+s"(iteration));  // keeps the first pass from being peeled into a copy
+      continue;
+    }
+    err[nw] = e_new;
     lde = wave_total(lde);
     const LmDecision d = lm_decide(err[init], err[nw], err[best], lde, lambda, nu, iteration, p,
                                    0, 0.0, 0.0, 0.0, eps);
     record(d.rec);
     lambda = d.lambda;
     nu = d.nu;
-    if (!d.accept) {
+    // the same in every lane: through readfirstlane the state blocks' indices stay scalar, and with
+    // them the addresses of their records
+    const int accept = __builtin_amdgcn_readfirstlane(d.accept);
+    const int set_best = __builtin_amdgcn_readfirstlane(d.set_best);
+    if (!accept) {
       const int s = nw;
       nw = init;
       init = s;
     } else {
-      if (d.set_best) {
+      if (set_best) {
         if (best != nw) {
           if (best != init) fre = best;
           best = nw;
@@ -425,9 +560,10 @@ batch_lm_kernel(BatchView v, symhip_optimizer_params p, double eps) {
         fre = best;
       }
     }
-    status = d.status;
+    status = __builtin_amdgcn_readfirstlane(d.status);
     reason = d.reason;
     done = status != 0;
+    ++iteration;
   }
   if (!done && status == 0) status = SYMHIP_STATUS_HIT_ITERATION_LIMIT;
   if (live)
@@ -507,6 +643,8 @@ BatchLocalization::BatchLocalization(const symhip_problem_desc* descs, int32_t n
   std::vector<int32_t>& pose_begin = pk.pose_begin;
   std::vector<double>& cvals = pk.cvals;
   total_poses_ = pose_begin.back();
+  for (int32_t i = 0; i < n_problems; ++i)
+    max_poses_ = std::max(max_poses_, pose_begin[i + 1] - pose_begin[i]);
   cvals_host_size_ = cvals.size();
   HIP_OK(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
   HIP_OK(hipEventCreate(&ev0_));
@@ -556,7 +694,8 @@ void BatchLocalization::build_graph(int c) {
   hipGraph_t graph;
   HIP_OK(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
   auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(n_problems_), dim3(64), 0, stream_, v, p_, eps_);
+    hipLaunchKernelGGL(kernel, dim3(n_problems_), dim3(64), rec_bytes(max_poses_), stream_, v, p_,
+                       eps_);
   };
   if (f32_) {
     if (c & 1) launch(batch_lm_kernel<float, 2>); else launch(batch_lm_kernel<float, 1>);
@@ -695,11 +834,11 @@ void batch_solve_noalloc(const symhip_batch_tables& t, const symhip_optimizer_pa
               t.odo_args,  t.values,     vals,        lin,                maxd,
               values_out,  iters_out,    p.iterations + 1, stats_out,     ticks, nullptr};
   if (precision == SYMHIP_PRECISION_F32_JAC)
-    hipLaunchKernelGGL((batch_lm_kernel<float, 1>), dim3(t.n_problems), dim3(64), 0, stream, v,
-                       p, epsilon);
+    hipLaunchKernelGGL((batch_lm_kernel<float, 1>), dim3(t.n_problems), dim3(64),
+                       rec_bytes(kMaxPoses), stream, v, p, epsilon);
   else
-    hipLaunchKernelGGL((batch_lm_kernel<double, 1>), dim3(t.n_problems), dim3(64), 0, stream, v,
-                       p, epsilon);
+    hipLaunchKernelGGL((batch_lm_kernel<double, 1>), dim3(t.n_problems), dim3(64),
+                       rec_bytes(kMaxPoses), stream, v, p, epsilon);
   HIP_OK(hipGetLastError());
 }
 

@@ -11,6 +11,7 @@
 #include <algorithm>
 
 #include "./chol_numeric.h"
+#include "./dpp.h"
 #include "./util.h"
 
 namespace symhip {
@@ -83,14 +84,6 @@ constexpr int kDiagRows = 2 * kMaxCols;    // diagonal block + one chunk of belo
 constexpr int kCbLd = kDiagRows + 4;       // cb[u][row]: published columns
 constexpr int kLcLd = kDiagRows + 2;       // Lc[col][row]: the working matrix, then L and D
 constexpr int kDiagSmem = kStep * kCbLd + kStep * kDiagRows + kMaxCols * kLcLd;
-
-// 1 / d by the hardware estimate and two Newton steps (the IEEE division sequence is twice as
-// long, and these sit on the sweep's critical path).
-__device__ __forceinline__ double refined_rcp(double d) {
-  double r = __builtin_amdgcn_rcp(d);
-  r = fma(r, fma(-d, r, 1.0), r);
-  return fma(r, fma(-d, r, 1.0), r);
-}
 
 // Step 2 for row t: cb[u][i] = A(i, k0 + u) after the previous steps; writes Wt[u][t] = w_u and
 // Lc[k0 + u][t] = L(t, k0 + u).
