@@ -51,82 +51,45 @@ __global__ void assemble_kernel(int64_t nnz, const int64_t* __restrict__ map,
 }
 
 // Diagonal task (s, chunk): one 512-thread block eliminates the 64 x 64 diagonal block of
-// supernode s together with the chunk's 64 below rows in one right-looking sweep of kStep-column
-// steps (the diagonal block is factored redundantly by every chunk of s; chunk 0 writes L11 to
-// l11 and D), leaving L21 = A21 L11^-T D^-1 for its rows, written back into the panel in place.
+// supernode s together with the chunk's 64 below rows and, with kFwd, the right-hand side as one
+// more row, in a right-looking sweep of 16-column panels (the diagonal block is factored
+// redundantly by every chunk of s; chunk 0 writes L11 to l11 and D), leaving L21 = A21 L11^-T D^-1
+// for its rows, written back into the panel in place.
 //
-// The 128 x 64 working matrix (rows 0..63 the diagonal block padded with identity, rows 64..127
-// the chunk's below rows) lives in matrix-core accumulators: wave w holds rows 16w .. 16w + 15 as
-// four 16 x 16 tiles. Step k0 = 0, kStep, .., 64 - kStep:
-//  1. the lanes holding columns k0 .. k0 + kStep - 1 publish them to cb (LDS; for k0 > 0 right
-//     after the previous step's products for those columns, before its other tiles');
-//  2. row owners (thread t < 128 owns row t) factor the kStep x kStep pivot block (redundantly,
-//     a chain of kStep reciprocals), form their row's w = c Lp^-T (c = the row's published
-//     entries, Lp the pivot block's unit lower factor) and L = w D^-1, and write w to Wt and L
-//     to Lc (the pivot rows get Lp and D instead);
-//  3. every wave applies A(i, j) -= sum_u L(i, u) w(j, u) to its live tiles with
-//     v_mfma_f64_16x16x4f64 (operands read straight from Lc and Wt).
-// Each row's elimination is computed once, and an update needs a few LDS reads per lane per step
-// (a register-patch FMA form read 16 per column, and was bound by them). The owner phase is a
-// dependent FP64 chain that grows with the cube of kStep per step: 4-column steps beat 8-column
-// ones (measured), the extra barriers notwithstanding. Tiles that are dead for the rest of the
-// sweep are skipped (the step loop is unrolled; the row test is wave-uniform): columns below
-// k0 + kStep and diagonal-block row tiles above it. Within live tiles nothing is masked: entries
-// above the diagonal and finished columns pick up products of other such entries but are never
-// read again (the final values are in Lc), and the entries still to be eliminated only ever
-// combine lower-triangle values.
+// The working matrix (rows 0..63 the diagonal block padded with identity, rows 64..127 the chunk's
+// below rows, row 128 the right-hand side) is in LDS, Lc[column][row]; its columns past the
+// current panel live in matrix-core accumulators: wave w holds rows 16w .. 16w + 15 as 16 x 16
+// tiles. Per panel:
+//  1. two wavefronts eliminate its 16 columns with a row per lane and no barrier inside
+//     (panel_columns): X the diagonal block's rows and the right-hand side, Y the below rows, each
+//     with its own copy of the pivot rows. The other waves meanwhile apply the previous panel to
+//     their later tiles;
+//  2. every wave applies A(i, j) -= sum_u L(i, u) w(j, u) (w = L D) to its tile of the next panel's
+//     columns with four v_mfma_f64_16x16x4f64, operands read from Lc and Wt, and puts the tile
+//     into Lc; the operands of its later tiles are fetched for step 1.
+// X and Y are waves whose own tiles are finished: the panel's pivot rows' and those before them.
+// Panels past the supernode's last column are skipped (the padding stays the identity, which its
+// elimination would not change).
+//
+// Bound by latency: with one task per CU a launch is 5.7 k cycles of descriptor and staging loads,
+// four panels (2.7 k each, the vector pipe full with the broadcasts and multiply-adds of 16 columns
+// on two rows a lane; the first one 2 k more, its code being fetched), three exchanges (1.3 k) and
+// 4.7 k for the right-hand side's products and the stores. Before, 4-column steps with two barriers
+// each (a pivot block formed by every row's owner, 16 LDS round trips and rank-4 products): per
+// launch 17.7 -> 15.8 us on the 1000-camera system, 16.8 -> 14.8 at 137 cameras, 38 -> 33 on the
+// 100 000-node pose graph (8 006 leaf tasks, two per CU). Leaving a panel early after 4, 8 or 12
+// columns spilled its registers; the pivot rows' entries through LDS or scalar lane reads were
+// slower (see panel_columns).
 constexpr int kDiagThreads = 512;
-constexpr int kStep = 4;                   // columns eliminated per sweep step (4 or 8)
+constexpr int kPanel = 16;                 // columns per panel
 constexpr int kDiagRows = 2 * kMaxCols;    // diagonal block + one chunk of below rows
-// LDS layouts, padded so the owners' row-wise writes, the publishing lanes' writes and the
-// matrix-core operand reads are free of bank conflicts (row-major arrays with 8-double rows cost
-// 16-way conflicts on the owners' writes, four fifths of the owner phase)
-constexpr int kCbLd = kDiagRows + 4;       // cb[u][row]: published columns
-constexpr int kLcLd = kDiagRows + 2;       // Lc[col][row]: the working matrix, then L and D
-constexpr int kDiagSmem = kStep * kCbLd + kStep * kDiagRows + kMaxCols * kLcLd;
-
-// Step 2 for row t: cb[u][i] = A(i, k0 + u) after the previous steps; writes Wt[u][t] = w_u and
-// Lc[k0 + u][t] = L(t, k0 + u).
-__device__ __forceinline__ void sweep_owner(int k0, int t, const double (*cb)[kCbLd],
-                                            double (*Wt)[kDiagRows], double (*Lc)[kLcLd]) {
-  double d[kStep], dinv[kStep], Lp[kStep][kStep];
-  // pivot block, column by column: with wp_uv = L_uv d_v (row u's, formed when column u starts),
-  // d_u = A_uu - sum_v wp_uv L_uv and L_ru = (A_ru - sum_v L_rv wp_uv) / d_u
-#pragma unroll
-  for (int u = 0; u < kStep; ++u) {
-    double wp[kStep];
-#pragma unroll
-    for (int v = 0; v < u; ++v) wp[v] = Lp[u][v] * d[v];
-    double dd = cb[u][k0 + u];
-#pragma unroll
-    for (int v = 0; v < u; ++v) dd -= wp[v] * Lp[u][v];
-    d[u] = dd;
-    dinv[u] = refined_rcp(dd);
-#pragma unroll
-    for (int r = u + 1; r < kStep; ++r) {
-      double x = cb[u][k0 + r];
-#pragma unroll
-      for (int v = 0; v < u; ++v) x -= Lp[r][v] * wp[v];
-      Lp[r][u] = x * dinv[u];
-    }
-  }
-  double w[kStep], l[kStep];
-#pragma unroll
-  for (int u = 0; u < kStep; ++u) {
-    double c = cb[u][t];
-#pragma unroll
-    for (int v = 0; v < u; ++v) c -= w[v] * Lp[u][v];
-    w[u] = c;
-    l[u] = c * dinv[u];
-  }
-  // pivot row k0 + r: Lp row left of the diagonal, D on it (w_r = d_r), zero right of it
-  const int r = t - k0;
-#pragma unroll
-  for (int u = 0; u < kStep; ++u) {
-    Wt[u][t] = w[u];
-    Lc[k0 + u][t] = (r < 0 || r >= kStep || u < r) ? l[u] : (u == r ? w[u] : 0.0);
-  }
-}
+constexpr int kRhsRow = kDiagRows;         // the right-hand side's row
+// LDS: two spare rows keep column starts off the same banks (and hold the right-hand side); two
+// blocks fit a CU (75.5 KB each)
+constexpr int kLcLd = kDiagRows + 2;       // Lc[col][row]
+constexpr int kWtLd = kMaxCols + 2;        // Wt[u][row]: w of the panel's columns
+constexpr int kWtRhs = kMaxCols;           // .. and of the right-hand side's row
+constexpr int kDiagSmem = kMaxCols * kLcLd + kPanel * kWtLd + kMaxCols;
 
 // Value of v in lane k (k wave-uniform), through two scalar lane reads: a short dependency for
 // the triangular recurrences (an LDS-based shuffle costs a full LDS round trip per step).
@@ -136,11 +99,48 @@ __device__ __forceinline__ double lane_value(double v, int k) {
                                               __builtin_amdgcn_readlane(u.y, k)));
 }
 
+template <int K, int J>
+__device__ __forceinline__ void panel_updates(double (&s0)[kPanel], double (&s1)[kPanel], double w,
+                                              double l0, double l1) {
+  if constexpr (J < kPanel) {
+    const double b = row_bcast<J>(w);
+    s0[J] = fma(-l0, b, s0[J]);
+    s1[J] = fma(-l1, b, s1[J]);
+    panel_updates<K, J + 1>(s0, s1, w, l0, l1);
+  }
+}
+
+// Columns K.. of a panel: s0 holds the pivot rows (row l % 16 in lane l, four copies), s1 a row per
+// lane. Column K: d = its pivot, l = own entry / d, and each later column j loses l w_j, w_j the
+// pivot row j's entry, which row_bcast brings from the lane's own row of 16 (a broadcast and two
+// multiply-adds, ~17 cycles; by scalar lane reads, or through LDS, the panel took 3.0-4.4 k cycles
+// against 2.8). s0 and s1 end as L, and every lane's s1 entry goes to put[K * kLcLd] as it is
+// formed; with kX its w goes to wput[K * kWtLd] too and pivot row r's lanes keep their d in dg.
+template <bool kX, int K = 0>
+__device__ __forceinline__ void panel_columns(double (&s0)[kPanel], double (&s1)[kPanel],
+                                              double* put, double* wput, int lr, double& dg) {
+  if constexpr (K < kPanel) {
+    const double w = s0[K], w1 = s1[K];
+    const double dinv = refined_rcp(row_bcast<K>(w));
+    if (kX) wput[K * kWtLd] = w1;
+    const double l0 = w * dinv, l1 = w1 * dinv;
+    panel_updates<K, K + 1>(s0, s1, w, l0, l1);
+    put[K * kLcLd] = l1;
+    if (kX) {
+      dg = lr == K ? w : dg;
+      s0[K] = l0;
+    }
+    // a column's instructions fill the vector pipe by themselves; mixing columns only costs registers
+    __builtin_amdgcn_sched_barrier(0);
+    panel_columns<kX, K + 1>(s0, s1, put, wput, lr, dg);
+  }
+}
+
 // Forward solve fused into the diagonal task (kFwd): with y = P b plus the updates of every
-// descendant (earlier levels), the block forms y_own = L11^-1 y_own (wave 0, lane r holding y_r)
-// once L11 is in LDS, chunk 0 writes it to yout, and the chunk's below rows get
-// y(row) -= L21(row, :) y_own atomically (siblings share ancestors). The same work as a separate
-// forward launch per level, without the launch.
+// descendant (earlier levels), the right-hand side's row leaves the sweep as w = L11^-1 y_own,
+// chunk 0 writes it to yout, and the chunk's below rows get y(row) -= L21(row, :) y_own atomically
+// (siblings share ancestors). The same work as a separate forward launch per level, without the
+// launch.
 template <bool kFwd>
 __device__ __forceinline__ void diag_body(const SnTask& tk, double* __restrict__ panel,
                                           double* __restrict__ l11,
@@ -148,9 +148,9 @@ __device__ __forceinline__ void diag_body(const SnTask& tk, double* __restrict__
                                           double* __restrict__ y, double* __restrict__ yout,
                                           double* smem) {
   typedef double d4 __attribute__((ext_vector_type(4)));
-  auto cb = reinterpret_cast<double (*)[kCbLd]>(smem);
-  auto Wt = reinterpret_cast<double (*)[kDiagRows]>(smem + kStep * kCbLd);
-  auto Lc = reinterpret_cast<double (*)[kLcLd]>(smem + kStep * kCbLd + kStep * kDiagRows);
+  auto Lc = reinterpret_cast<double (*)[kLcLd]>(smem);
+  auto Wt = reinterpret_cast<double (*)[kWtLd]>(smem + kMaxCols * kLcLd);
+  double* zs = smem + kMaxCols * kLcLd + kPanel * kWtLd;  // the solved right-hand side
   const SnDesc sd = tk.d;
   const int chunk = tk.a;
   const int n = sd.ncols, ld = sd.ld, mb = ld - n;
@@ -190,110 +190,179 @@ __device__ __forceinline__ void diag_body(const SnTask& tk, double* __restrict__
     const double fill = (!below & (i == j)) ? 1.0 : 0.0;
     Lc[j][i] = keep ? v[q] : fill;
   }
+  if (wave == 0) {
+    Lc[lane][kRhsRow] = kFwd && lane < n ? y_in : 0.0;
+    zs[lane] = 0.0;
+  }
   __syncthreads();
-  // Wave w holds rows 16w .. 16w + 15 as four 16 x 16 accumulator tiles (columns 16c ..), in the
-  // v_mfma_f64_16x16x4f64 layout: acc[c][r] = A(16w + lane / 16 + 4r, 16c + lane % 16).
-  d4 acc[4];
+  // acc[t] holds the tile of columns 16 (p + 1 + t) .. for the current panel p, in the
+  // v_mfma_f64_16x16x4f64 layout: acc[t][r] = A(16w + lane / 16 + 4r, 16 (p + 1 + t) + lane % 16).
+  // A tile above the diagonal block's diagonal is never read: waves 0..3 keep columns up to 16w.
+  constexpr int kTiles = kMaxCols / kPanel - 1;
+  d4 acc[kTiles] = {};
+  auto load_tiles = [&] {
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
+    for (int t = 0; t < kTiles; ++t)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) acc[c][r] = Lc[16 * c + lr][16 * wave + lk + 4 * r];
-  // (the first barrier of the sweep orders these reads before the owners' Lc writes)
-  const bool below_wave = wave >= kMaxCols / 16;
-  // Steps past the supernode's last column are skipped (the padding stays the identity, which
-  // its elimination would not change): a 6-column supernode takes 2 steps, not 16. (Skipping the
-  // padding's MFMA tiles, or ending the solve chains at n, measured slower: the extra runtime
-  // conditions cost the unrolled loops their schedule.)
-  // publish columns k0 .. k0 + kStep - 1 (tile column k0 / 16, lanes k0 % 16 ..) of the rows
-  // from k0 on
-  auto publish = [&](int k0) {
-    const int off = k0 & 15, cp = k0 >> 4;
-    if ((below_wave || 16 * wave + 15 >= k0) && lr >= off && lr < off + kStep) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) cb[lr - off][16 * wave + lk + 4 * r] = acc[cp][r];
-    }
+      for (int r = 0; r < 4; ++r)
+        acc[t][r] = Lc[kPanel * (1 + t) + lr][16 * wave + lk + 4 * r];
   };
-  publish(0);
+  if (wave >= 2) load_tiles();
+  // operands of the later tiles, from one panel's step 2 to the next one's step 1
+  double av[4], bv[kTiles - 1][4];
 #pragma unroll
-  for (int st = 0; st < kMaxCols / kStep; ++st) {
-    const int k0 = kStep * st;
-    if (k0 >= n) break;
-    __syncthreads();
-    if (tid < kDiagRows) sweep_owner(k0, tid, cb, Wt, Lc);
-    __syncthreads();
-    const int kn = k0 + kStep;  // first column still to be eliminated
-    if (kn < kMaxCols && (below_wave || 16 * wave + 15 >= kn)) {
-      // A(i, j) -= sum_u L(i, k0 + u) w(j, u) on the matrix cores, kStep / 4 K = 4 pieces per tile:
-      // lane l feeds A(l % 16, l / 16) = -L(16w + l % 16, k0 + 4h + l / 16) and
-      // B(l / 16, l % 16) = w(16c + l % 16, 4h + l / 16)
-      double av[kStep / 4];
+  for (int h = 0; h < 4; ++h) av[h] = bv[0][h] = bv[1][h] = 0.0;
+  for (int k0 = 0;; k0 += kPanel) {
+    const int p = k0 / kPanel;
+    const int wx = p, wy = p == 0 ? 1 : p - 1;
+    // The panel's own waves run at a higher priority than the tile waves on their SIMDs: they are
+    // the block's critical path.
+    if (wave == wx) {
+      // lanes: rows 16 .. 63 of the diagonal block, then the right-hand side; rows up to the
+      // panel's pivots are finished, eliminated along and stored to the spare row
+      const int row = lane < kMaxCols - kPanel ? kPanel + lane : kRhsRow;
+      __builtin_amdgcn_s_setprio(2);
+      double s0[kPanel], s1[kPanel], dg = 0.0;
 #pragma unroll
-      for (int h = 0; h < kStep / 4; ++h) av[h] = -Lc[k0 + 4 * h + lk][16 * wave + lr];
-      // The tile of the next step's pivot columns first, published at once (the owners of this
-      // step are done with cb); the other tiles' products then run behind the next step's
-      // barrier and owner phase (measured: 16.4 -> 16.0 us per diagonal launch).
-      const int cpn = kn >> 4;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        if (c != cpn) continue;
-#pragma unroll
-        for (int h = 0; h < kStep / 4; ++h)
-          acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[h], Wt[4 * h + lk][16 * c + lr], acc[c],
-                                                         0, 0, 0);
+      for (int u = 0; u < kPanel; ++u) {
+        s0[u] = Lc[k0 + u][k0 + lr];
+        s1[u] = Lc[k0 + u][row];
       }
-      if (kn < n) publish(kn);
+      panel_columns<true>(s0, s1, &Lc[k0][row < k0 + kPanel ? kRhsRow + 1 : row],
+                          &Wt[0][row == kRhsRow ? kWtRhs : row], lr, dg);
+      __builtin_amdgcn_s_setprio(0);
+      __syncthreads();
+      if (lane < kPanel) {
+        // the pivot rows, which Y has read by now: L, D on the diagonal, zeros right of it
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        if (c == cpn || 16 * c + 15 < kn) continue;  // done above / columns already eliminated
+        for (int u = 0; u < kPanel; ++u)
+          Lc[k0 + u][k0 + lane] = u < lane ? s0[u] : (u == lane ? dg : 0.0);
+        if (kFwd) zs[k0 + lane] = Wt[lane][kWtRhs];
+      }
 #pragma unroll
-        for (int h = 0; h < kStep / 4; ++h)
-          acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[h], Wt[4 * h + lk][16 * c + lr], acc[c],
-                                                         0, 0, 0);
+      for (int t = 0; t < kTiles; ++t) acc[t] = d4{};  // finished: not live across the panel
+    } else if (wave == wy) {
+      __builtin_amdgcn_s_setprio(2);
+      double s0[kPanel], s1[kPanel], dg = 0.0;
+#pragma unroll
+      for (int u = 0; u < kPanel; ++u) {
+        s0[u] = Lc[k0 + u][k0 + lr];
+        s1[u] = Lc[k0 + u][kMaxCols + lane];
+      }
+      panel_columns<false>(s0, s1, &Lc[k0][kMaxCols + lane], nullptr, lr, dg);
+      __builtin_amdgcn_s_setprio(0);
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t) acc[t] = d4{};
+      if (p == 0) load_tiles();
+    } else {
+      if (k0 > 0) {
+#pragma unroll
+        for (int t = 1; t < kTiles; ++t) {
+#pragma unroll
+          for (int h = 0; h < 4; ++h)
+            acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[h], bv[t - 1][h], acc[t], 0, 0, 0);
+          acc[t - 1] = acc[t];
+        }
+      }
+      __syncthreads();
+    }
+    const int kn = k0 + kPanel;  // first column still to be eliminated
+    if (kn >= n) break;          // uniform
+    if (wave > p) {
+      // A(i, j) -= sum_u L(i, k0 + u) w(j, u): lane l feeds A(l % 16, l / 16) =
+      // -L(16w + l % 16, k0 + 4h + l / 16) and B(l / 16, l % 16) = w(16c + l % 16, 4h + l / 16)
+      double bn[4];
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        av[h] = -Lc[k0 + 4 * h + lk][16 * wave + lr];
+        bn[h] = Wt[4 * h + lk][kn + lr];
+      }
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+        acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[h], bn[h], acc[0], 0, 0, 0);
+#pragma unroll
+      for (int t = 1; t < kTiles; ++t)
+#pragma unroll
+        for (int h = 0; h < 4; ++h)  // past the last tile: clamped, its accumulator is not used
+          bv[t - 1][h] = Wt[4 * h + lk][min(kn + kPanel * t, kMaxCols - kPanel) + lr];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) Lc[kn + lr][16 * wave + lk + 4 * r] = acc[0][r];
+    } else {
+#pragma unroll
+      for (int h = 0; h < 4; ++h) av[h] = bv[0][h] = bv[1][h] = 0.0;
+    }
+    if (kFwd && wave == (p == 0 ? 0 : p - 1)) {  // a wave without tiles, X's stores aside
+      // the right-hand side's later columns: y_j -= sum_u l_y w_j
+      const int j = kn + lane;
+      if (j < kMaxCols) {
+        double t = Lc[j][kRhsRow];
+#pragma unroll
+        for (int u = 0; u < kPanel; ++u) t = fma(-Lc[k0 + u][kRhsRow], Wt[u][j], t);
+        Lc[j][kRhsRow] = t;
       }
     }
+    __syncthreads();
   }
   __syncthreads();
-  if (kFwd && wave == 0) {
-    const int r = lane;
-    double yi = r < n ? y_in : 0.0;
+  if (kFwd) {
+    // L21 y_own, 16 columns by each of four waves, then added up by the first
+    auto part = reinterpret_cast<double (*)[kMaxCols]>(&Wt[0][0]);
+    if (wave < 4) {
+      double t = 0.0;
 #pragma unroll
-    for (int k = 0; k < kMaxCols; ++k) yi -= (r > k ? Lc[k][r] : 0.0) * lane_value(yi, k);
-    if (chunk == 0 && r < n) yout[sd.col_begin + r] = yi;
-    double acc = 0.0;
-#pragma unroll
-    for (int k = 0; k < kMaxCols; ++k) acc += Lc[k][kMaxCols + r] * lane_value(yi, k);
-    if (chunk * kMaxCols + r < mb) unsafeAtomicAdd(&y[y_row], -acc);
-    return;
-  }
-  // Write back with coalesced stores (with the forward solve, wave 0 is busy with it and the
-  // other waves store): L11 (strict lower, column-major n x n) and D from chunk 0, the chunk's
-  // L21 rows into the panel. The thread index passes through an empty asm so the compiler
-  // recomputes these addresses here instead of holding the load phase's across the sweep.
-  constexpr int kStorers = kFwd ? kDiagThreads - 64 : kDiagThreads;
-  int tid_w = kFwd ? tid - 64 : tid;
-  asm volatile("" : "+v"(tid_w));
-#pragma unroll 4
-  for (int idx = tid_w; idx < kDiagRows * kMaxCols; idx += kStorers) {
-    const int i = idx & (kDiagRows - 1), j = idx / kDiagRows;
-    const double v = Lc[j][i];
-    if (i < kMaxCols) {
-      if (chunk == 0 && i < n && j < n) {
-        if (i > j) l11[sd.l11_off + (int64_t)j * n + i] = v;
-        if (i == j) D[sd.col_begin + i] = v;
+      for (int u = 0; u < kPanel; ++u) {
+        const int k = kPanel * wave + u;
+        t = fma(Lc[k][kMaxCols + lane], zs[k], t);
       }
-    } else {
-      const int r = chunk * kMaxCols + i - kMaxCols;
-      if (r < mb && j < n) P[(int64_t)j * ld + n + r] = v;
+      part[wave][lane] = t;
+    }
+    __syncthreads();
+    if (wave == 0) {
+      if (chunk == 0 && lane < n) yout[sd.col_begin + lane] = zs[lane];
+      if (chunk * kMaxCols + lane < mb)
+        unsafeAtomicAdd(&y[y_row],
+                        -((part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane])));
+    }
+  }
+  // Write back with coalesced stores: L11 (strict lower, column-major n x n) and D from chunk 0
+  // (the even waves), the chunk's L21 rows into the panel (the odd ones); a wave takes every fourth
+  // column. The thread index passes through an empty asm so the compiler recomputes these
+  // addresses here instead of holding the load phase's across the sweep.
+  int tid_w = tid;
+  asm volatile("" : "+v"(tid_w));
+  const int i = tid_w & (kDiagRows - 1);
+  const int j0 = __builtin_amdgcn_readfirstlane(tid_w / kDiagRows);
+  constexpr int kStride = kDiagThreads / kDiagRows;
+  // (four columns a turn: the code is fetched for the first time here, and a fully unrolled copy of
+  // all sixteen is slower for it)
+  if (wave & 1) {
+    const int r = chunk * kMaxCols + i - kMaxCols;
+    double* dst = P + (int64_t)j0 * ld + n + r;
+    const int64_t step = (int64_t)kStride * ld;
+    if (r < mb) {
+#pragma unroll 4
+      for (int j = j0; j < n; j += kStride, dst += step) *dst = Lc[j][i];
+    }
+  } else if (chunk == 0) {
+    double* dst = l11 + sd.l11_off + (int64_t)j0 * n + i;
+    const int64_t step = (int64_t)kStride * n;
+    if (i < n) {
+#pragma unroll 4
+      for (int j = j0; j < n; j += kStride, dst += step)
+        if (i > j) *dst = Lc[j][i];
+      if ((i & (kStride - 1)) == j0) D[sd.col_begin + i] = Lc[i][i];
     }
   }
 }
 
 template <bool kFwd>
-__global__ void __launch_bounds__(kDiagThreads) diag_trsm_kernel(
+__global__ void __launch_bounds__(kDiagThreads) __attribute__((amdgpu_waves_per_eu(4)))
+diag_trsm_kernel(
     const SnTask* __restrict__ tasks, double* __restrict__ panel, double* __restrict__ l11,
     double* __restrict__ D, const int32_t* __restrict__ rows, double* __restrict__ y,
     double* __restrict__ yout) {
-  __shared__ double smem[kDiagSmem];
+  __shared__ __attribute__((aligned(16))) double smem[kDiagSmem];
   diag_body<kFwd>(tasks[blockIdx.x], panel, l11, D, rows, y, yout, smem);
 }
 
