@@ -13,13 +13,17 @@ namespace symhip {
 // tile kernels over supernodal panels, level by level in the supernodal elimination tree.
 class SupernodalLDLT {
  public:
-  // colptr/rowind: lower CSC pattern (host) of the matrices that will be factorized.
+  // colptr/rowind: lower CSC pattern (host) of the matrices that factorize() will be given; null
+  // where the caller writes the panels itself (factorize_assembled).
   void setup(const CholSymbolic& sym, const int32_t* colptr, const int32_t* rowind,
              hipStream_t s);
-  // Assembles A (device values in the CSC order given to setup) into panels and factorizes.
+  // Assembles A (device values in the CSC order given to setup) into panels and factorizes; with
+  // damping (device, original order), A + diag(damping). Captured in a hipGraph per argument list
+  // and replayed.
   // With b (device, original order) the forward solve L y = P b runs inside the factorization's
   // diagonal kernels, and solve_fused finishes x = A^-1 b.
-  void factorize(const double* a_values, hipStream_t s, const double* b = nullptr);
+  void factorize(const double* a_values, hipStream_t s, const double* b = nullptr,
+                 const double* damping = nullptr);
   // Panels already assembled by the caller (e.g. the Schur path writes them directly). The
   // per-level launch sequence is captured in a hipGraph per b on the first call and replayed.
   void factorize_assembled(hipStream_t s, const double* b = nullptr);
@@ -34,8 +38,9 @@ class SupernodalLDLT {
   void reserve_many(int32_t nrhs, hipStream_t s);
   int32_t many_capacity(int32_t nrhs) const;
   static constexpr int64_t kManyBytes = 256 << 20;
-  // x = A^-1 b for the b given to the last factorization (backward half only); x may alias b.
-  void solve_fused(double* x, hipStream_t s);
+  // x = A^-1 b for the b given to the last factorization (backward half only), or -A^-1 b with
+  // negate; x may alias b.
+  void solve_fused(double* x, hipStream_t s, bool negate = false);
   SupernodalLDLT() = default;
   SupernodalLDLT(const SupernodalLDLT&) = delete;
   SupernodalLDLT& operator=(const SupernodalLDLT&) = delete;
@@ -55,22 +60,28 @@ class SupernodalLDLT {
   // permutation): strictly lower unit L, from the factored diagonal blocks and the panels.
   void factor_values(const std::vector<int32_t>& l_colptr, const std::vector<int32_t>& l_rowind,
                      double* values, hipStream_t s) const;
-  int64_t assembly_nnz() const { return (int64_t)asm_map_.size(); }
 
  private:
   void launch_factorize(const double* b, hipStream_t s);
   void launch_solve(const double* b, double* x, hipStream_t s);
-  void launch_backward(double* x, hipStream_t s);
+  void launch_backward(double* x, double sign, hipStream_t s);
+  struct GraphInputs {
+    const double* vals = nullptr;
+    const double* damping = nullptr;
+    const double* b = nullptr;
+    bool operator==(const GraphInputs&) const = default;
+  };
   struct CachedGraph {
-    const double* b;
+    GraphInputs in;
     double* x;
+    double sign;
     bool f32;  // factorization graphs: the update form captured
     hipGraphExec_t exec;
   };
   template <typename F>
-  hipGraphExec_t cached_graph(std::vector<CachedGraph>& cache, const double* b, double* x,
-                              hipStream_t s, F&& launches);
-  // captured launch sequences, one per argument pair seen (a few state blocks)
+  hipGraphExec_t cached_graph(std::vector<CachedGraph>& cache, const GraphInputs& in, double* x,
+                              double sign, hipStream_t s, F&& launches);
+  // captured launch sequences, one per argument list seen (a few state blocks)
   std::vector<CachedGraph> fact_graphs_, solve_graphs_, bwd_graphs_;
   bool fused_ = false;  // the last factorization ran the forward solve
   bool f32_updates_ = false;
@@ -79,7 +90,8 @@ class SupernodalLDLT {
   DBuf<int32_t> counter_;  // per-supernode arrival counters of the backward pass (self-resetting)
   DBuf<double> many_y_, many_yout_, many_part_;  // solve_many
   DBuf<int32_t> many_counter_;                   // per (right-hand-side group, supernode)
-  DBuf<int64_t> asm_map_, scat_col_;
+  DBuf<int64_t> scat_col_;
+  DBuf<int32_t> panel_src_, diag_pos_;  // factorize(): what each panel entry is assembled from
   DBuf<int32_t> rows_, perm_, upd_rel_, scat_rel_;
   DBuf<uint8_t> trsm_tasks_, upd_tasks_, solve_tasks_;  // per-level task lists (chol_numeric.hip)
   // work lists (flattened over levels)

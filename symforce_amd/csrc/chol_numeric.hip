@@ -4,9 +4,8 @@
 // cores, set_f32_updates).
 //
 // The work per supernode is small (panels are at most 64 columns wide), so every kernel is
-// latency-bound: the kernels are written to avoid data-dependent branches (the 64 elimination
-// steps are fully unrolled over a panel padded to 64 columns, the padding being an identity
-// block) and chains of dependent global loads (each supernode's metadata is one descriptor,
+// latency-bound: the kernels are written to avoid data-dependent branches (16 elimination steps
+// are unrolled over panels padded to 64 columns, the padding being an identity block) and chains of dependent global loads (each supernode's metadata is one descriptor,
 // scatter targets are precomputed per below-row).
 #include <algorithm>
 
@@ -43,11 +42,30 @@ struct SnTask {
   int32_t s, a, b, pad;  // supernode; chunk or tile row; tile column
 };
 
-__global__ void assemble_kernel(int64_t nnz, const int64_t* __restrict__ map,
-                                const double* __restrict__ vals, double* __restrict__ panel) {
-  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < nnz;
-       q += (int64_t)gridDim.x * blockDim.x)
-    panel[map[q]] = vals[q];
+// The panels of A + diag(damping) (damping null: of A), every entry written once: bound by the
+// panel's 12 bytes per entry. Zeroing the panels and scattering the matrix into them took two
+// launches and wrote its lines twice.
+__global__ void __launch_bounds__(256) assemble_kernel(int64_t size,
+                                                       const int32_t* __restrict__ src,
+                                                       const int32_t* __restrict__ diag,
+                                                       const double* __restrict__ vals,
+                                                       const double* __restrict__ damping,
+                                                       double* __restrict__ panel) {
+  const int64_t i = 2 * (blockIdx.x * (int64_t)256 + threadIdx.x);
+  if (i >= size) return;
+  auto value = [&](int32_t c) __attribute__((always_inline)) {
+    if (c >= 0) return vals[c];
+    if (c == kPanelFill) return 0.0;
+    const int32_t j = -2 - c;
+    const double v = vals[diag[j]];
+    return damping ? v + damping[j] : v;
+  };
+  if (i + 1 < size) {  // the buffers' own bases and an even i: aligned pairs
+    const int2 c = *reinterpret_cast<const int2*>(src + i);
+    *reinterpret_cast<double2*>(panel + i) = make_double2(value(c.x), value(c.y));
+  } else {
+    panel[i] = value(src[i]);
+  }
 }
 
 // Diagonal task (s, chunk): one 512-thread block eliminates the 64 x 64 diagonal block of
@@ -512,9 +530,10 @@ __global__ void permute_kernel(int32_t n, const int32_t* __restrict__ perm,
   }
 }
 __global__ void unpermute_kernel(int32_t n, const int32_t* __restrict__ perm,
-                                 const double* __restrict__ y, double* __restrict__ x) {
+                                 const double* __restrict__ y, double sign,
+                                 double* __restrict__ x) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) x[i] = y[perm[i]];
+  if (i < n) x[i] = sign * y[perm[i]];
 }
 
 // Stages the strictly lower part of L11 (n x n column-major at Lc, padded with zeros; unit
@@ -897,9 +916,13 @@ void SupernodalLDLT::setup(const CholSymbolic& sym, const int32_t* colptr, const
                            hipStream_t s) {
   SYMHIP_CHECK(sym.max_snode_cols <= kMaxCols, "supernode wider than the kernel tile");
   sym_ = sym;
-  std::vector<int64_t> map = chol_assembly_map(sym, colptr, rowind);
-  asm_map_.upload(map, s);
   panel_.resize(std::max<int64_t>(1, sym.panel_size()));
+  std::vector<int32_t> src, diag;
+  if (colptr) {
+    chol_panel_sources(sym, colptr, rowind, src, diag);
+    panel_src_.upload(src, s);
+    diag_pos_.upload(diag, s);
+  }
   D_.resize(std::max(1, sym.n));
   y_.resize(std::max(1, sym.n));
   yout_.resize(std::max(1, sym.n));
@@ -998,15 +1021,16 @@ void SupernodalLDLT::setup(const CholSymbolic& sym, const int32_t* colptr, const
   HIP_OK(hipStreamSynchronize(s));
 }
 
-void SupernodalLDLT::factorize(const double* a_values, hipStream_t s, const double* b) {
-  fill_zero(panel_.get(), sym_.panel_size(), s);
-  const int64_t nnz = (int64_t)asm_map_.size();
-  if (nnz) {
-    const int grid = (int)std::min<int64_t>(grid_for(nnz, 256), 8192);
-    hipLaunchKernelGGL(assemble_kernel, dim3(grid), dim3(256), 0, s, nnz, asm_map_.get(), a_values,
-                       panel_.get());
-  }
-  factorize_assembled(s, b);
+void SupernodalLDLT::factorize(const double* a_values, hipStream_t s, const double* b,
+                               const double* damping) {
+  if (sym_.n_levels == 0) return;
+  fused_ = b != nullptr;
+  HIP_OK(hipGraphLaunch(cached_graph(fact_graphs_, {a_values, damping, b}, nullptr, 1.0, s, [&] {
+    const int64_t size = sym_.panel_size();
+    hipLaunchKernelGGL(assemble_kernel, dim3(grid_for(size, 512)), dim3(256), 0, s, size,
+                       panel_src_.get(), diag_pos_.get(), a_values, damping, panel_.get());
+    launch_factorize(b, s);
+  }), s));
 }
 
 SupernodalLDLT::~SupernodalLDLT() {
@@ -1031,13 +1055,14 @@ hipGraphExec_t capture(hipStream_t s, F&& launches) {
 void SupernodalLDLT::factorize_assembled(hipStream_t s, const double* b) {
   if (sym_.n_levels == 0) return;
   fused_ = b != nullptr;
-  HIP_OK(hipGraphLaunch(cached_graph(fact_graphs_, b, nullptr, s,
+  HIP_OK(hipGraphLaunch(cached_graph(fact_graphs_, {nullptr, nullptr, b}, nullptr, 1.0, s,
                                      [&] { launch_factorize(b, s); }), s));
 }
 
 void SupernodalLDLT::solve(const double* b, double* x, hipStream_t s) {
   if (sym_.n == 0) return;
-  HIP_OK(hipGraphLaunch(cached_graph(solve_graphs_, b, x, s, [&] { launch_solve(b, x, s); }), s));
+  HIP_OK(hipGraphLaunch(cached_graph(solve_graphs_, {nullptr, nullptr, b}, x, 1.0, s,
+                                     [&] { launch_solve(b, x, s); }), s));
 }
 
 int32_t SupernodalLDLT::many_capacity(int32_t nrhs) const {
@@ -1086,23 +1111,24 @@ void SupernodalLDLT::solve_many(const double* b, double* x, int32_t nrhs, hipStr
   HIP_OK(hipGetLastError());
 }
 
-void SupernodalLDLT::solve_fused(double* x, hipStream_t s) {
+void SupernodalLDLT::solve_fused(double* x, hipStream_t s, bool negate) {
   if (sym_.n == 0) return;
   SYMHIP_CHECK(fused_, "solve_fused needs a factorization given the right-hand side");
-  HIP_OK(hipGraphLaunch(cached_graph(bwd_graphs_, nullptr, x, s, [&] { launch_backward(x, s); }),
-                        s));
+  const double sign = negate ? -1.0 : 1.0;
+  HIP_OK(hipGraphLaunch(cached_graph(bwd_graphs_, {}, x, sign, s,
+                                     [&] { launch_backward(x, sign, s); }), s));
 }
 
 template <typename F>
-hipGraphExec_t SupernodalLDLT::cached_graph(std::vector<CachedGraph>& cache, const double* b,
-                                            double* x, hipStream_t s, F&& launches) {
+hipGraphExec_t SupernodalLDLT::cached_graph(std::vector<CachedGraph>& cache, const GraphInputs& in,
+                                            double* x, double sign, hipStream_t s, F&& launches) {
   for (const auto& g : cache)
-    if (g.b == b && g.x == x && g.f32 == f32_updates_) return g.exec;
+    if (g.in == in && g.x == x && g.sign == sign && g.f32 == f32_updates_) return g.exec;
   if (cache.size() >= 8) {  // bound the cache; the oldest goes
     (void)hipGraphExecDestroy(cache.front().exec);
     cache.erase(cache.begin());
   }
-  cache.push_back({b, x, f32_updates_, capture(s, launches)});
+  cache.push_back({in, x, sign, f32_updates_, capture(s, launches)});
   return cache.back().exec;
 }
 
@@ -1145,12 +1171,12 @@ void SupernodalLDLT::launch_solve(const double* b, double* x, hipStream_t s) {
                        tasks + lvl_solve_ptr_[l], rows_.get(),
                        panel_.get(), l11_.get(), y_.get(), yout_.get());
   }
-  launch_backward(x, s);
+  launch_backward(x, 1.0, s);
 }
 
-// The backward levels (D^-1 folded in) and the inverse permutation, from the forward result in
-// yout.
-void SupernodalLDLT::launch_backward(double* x, hipStream_t s) {
+// The backward levels (D^-1 folded in) and the inverse permutation (times sign), from the forward
+// result in yout.
+void SupernodalLDLT::launch_backward(double* x, double sign, hipStream_t s) {
   const int n = sym_.n;
   const SnTask* tasks = reinterpret_cast<const SnTask*>(solve_tasks_.get());
   for (int l = sym_.n_levels - 1; l >= 0; --l) {
@@ -1161,7 +1187,7 @@ void SupernodalLDLT::launch_backward(double* x, hipStream_t s) {
                        counter_.get());
   }
   hipLaunchKernelGGL(unpermute_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, n, perm_.get(),
-                     yout_.get(), x);
+                     yout_.get(), sign, x);
   HIP_OK(hipGetLastError());
 }
 

@@ -186,6 +186,18 @@ SYMHIP_HD void rot3_retract_inplace(double* q, const double* w, double eps) {
   q[3] = r.w;
 }
 
+// Storage and tangent size of the types other than Rot3 and Pose3.
+SYMHIP_HD int vector_dim(int type) {
+  return type == SYMHIP_TYPE_SCALAR    ? 1
+         : type == SYMHIP_TYPE_VECTOR2  ? 2
+         : type == SYMHIP_TYPE_VECTOR3  ? 3
+         : type == SYMHIP_TYPE_VECTOR4  ? 4
+         : type == SYMHIP_TYPE_VECTOR5  ? 5
+         : type == SYMHIP_TYPE_VECTOR6  ? 6
+         : type == SYMHIP_TYPE_MATRIX33 ? 9
+                                        : 36;
+}
+
 // Values::Retract of one key (opt/values.cc:294-327, gen/cpp/sym/ops/pose3/lie_group_ops.cc:69-102):
 // Pose3 rotates on the right and translates additively, Rot3 rotates on the right, every vector
 // and matrix type adds its tangent (storage) entries.
@@ -198,14 +210,7 @@ SYMHIP_HD void retract_value(int type, double* v, const double* d, double eps) {
   } else if (type == SYMHIP_TYPE_ROT3) {
     rot3_retract_inplace(v, d, eps);
   } else {
-    const int td = type == SYMHIP_TYPE_SCALAR    ? 1
-                   : type == SYMHIP_TYPE_VECTOR2  ? 2
-                   : type == SYMHIP_TYPE_VECTOR3  ? 3
-                   : type == SYMHIP_TYPE_VECTOR4  ? 4
-                   : type == SYMHIP_TYPE_VECTOR5  ? 5
-                   : type == SYMHIP_TYPE_VECTOR6  ? 6
-                   : type == SYMHIP_TYPE_MATRIX33 ? 9
-                                                  : 36;
+    const int td = vector_dim(type);
     for (int k = 0; k < td; ++k) v[k] += d[k];
   }
 }

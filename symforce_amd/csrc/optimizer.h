@@ -33,13 +33,13 @@ struct SolverOptions {
 class SystemBackend {
  public:
   virtual ~SystemBackend() = default;
-  // Relinearize block b at device values; writes residual(b), the system and err (device scalar).
-  virtual void relinearize(int b, const double* values, double* err_out, hipStream_t s) = 0;
-  // Damp block b's Hessian diagonal (DampHessian, levenberg_marquardt_solver.tcc:22-54); writes
-  // damping (N) and keeps the undamped diagonal for restore().
+  // Relinearize block b at device values; writes residual(b) and the system.
+  virtual void relinearize(int b, const double* values, hipStream_t s) = 0;
+  // Damping of block b's Hessian diagonal (DampHessian, levenberg_marquardt_solver.tcc:22-54):
+  // writes damping (N) and the undamped diagonal; the Hessian keeps its values (solve() adds the
+  // damping as it assembles).
   virtual void damp(int b, const double* lambda_dev, const symhip_optimizer_params& p,
                     bool have_max_diagonal, hipStream_t s) = 0;
-  virtual void restore(int b, hipStream_t s) = 0;
   // update = -H^-1 rhs for block b (factorize + solve), in the reference state order.
   virtual void solve(int b, double* update, hipStream_t s) = 0;
   virtual const double* rhs(int b) const = 0;
@@ -202,11 +202,12 @@ class DeviceOptimizer {
   hipStream_t stream_ = nullptr;
   std::unique_ptr<SystemBackend> backend_;
   DBuf<double> values_[3];
-  DBuf<double> update_, last_update_, partials_;
+  DBuf<double> update_, last_update_, partials_, bold_partials_;
   DBuf<int32_t> retract_type_, retract_soff_, retract_toff_;
   LmDevState* dstate_ = nullptr;  // device
-  LmDevState* hstate_ = nullptr;  // pinned host mirror
+  LmDevState* hstate_ = nullptr;  // pinned host mirror, written by the finishing kernels
   int init_ = 0, new_ = 1, best_ = 0, free_ = 2;
+  // the block's whole Values storage is this run's (a step writes the optimized keys only)
   bool valid_[3] = {false, false, false};
   bool linearized_[3] = {false, false, false};
   bool have_max_diagonal_ = false, have_last_update_ = false;

@@ -206,60 +206,43 @@ __global__ void factor_check_kernel(int32_t n, const int32_t* __restrict__ type,
   bad[f] = factor_finite_upto<1>(type[f], a) ? 0 : 1;
 }
 
-// Record the iteration -1 statistics (levenberg_marquardt_solver.tcc:158-186).
-__global__ void lm_first_record_kernel(LmDevState* st, int init) {
-  st->rec = symhip_iteration_stats{};
-  st->rec.iteration = -1;
-  st->rec.new_error = st->err[init];
-  st->rec.current_lambda = st->lambda;
-  st->status = isfinite(st->err[init]) ? 0 : SYMHIP_STATUS_FAILED;
-  st->reason = isfinite(st->err[init]) ? 0 : SYMHIP_FAILURE_INITIAL_ERROR_NOT_FINITE;
-}
-
-// The accept / reject / lambda logic of Iterate (levenberg_marquardt_solver.tcc:239-340).
-__global__ void lm_decide_kernel(LmDevState* st, int init, int nw, int best, int iteration,
-                                 symhip_optimizer_params p, int have_last_update, double eps) {
-  const LmDecision d = lm_decide(st->err[init], st->err[nw], st->err[best], st->lde, st->lambda,
-                                 st->nu, iteration, p, have_last_update, st->nl2, st->nu2,
-                                 st->dotlu, eps);
-  st->rec = d.rec;
-  st->lambda = d.lambda;
-  st->nu = d.nu;
-  st->status = d.status;
-  st->reason = d.reason;
-  st->accept = d.accept;
-  st->set_best = d.set_best;
-}
-
 // Values::Retract over the optimized keys (opt/values.cc:314-327).
+// from the Init block into the New one, whose other keys hold their constants already.
 __global__ void retract_kernel(int32_t n, const int32_t* __restrict__ type,
                                const int32_t* __restrict__ soff, const int32_t* __restrict__ toff,
-                               const double* __restrict__ update, double* __restrict__ values,
-                               double eps) {
+                               const double* __restrict__ update, const double* __restrict__ from,
+                               double* __restrict__ to, double eps) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  retract_value(type[i], values + soff[i], update + toff[i], eps);
+  const int t = type[i], o = soff[i];
+  const int dim = t == SYMHIP_TYPE_POSE3 ? 7 : t == SYMHIP_TYPE_ROT3 ? 4 : vector_dim(t);
+  for (int k = 0; k < dim; ++k) to[o + k] = from[o + k];
+  retract_value(t, to + o, update + toff[i], eps);
 }
 
-// sum_i u_i (rhs_i - damping_i u_i)  (Linearization::LinearDeltaError, linearization.h:62-67),
+// The iteration's reductions, first pass, in one launch. Blocks below nr: partials of
+// sum residual^2 (Linearization::Error, opt/linearization.h:51-54) into part. The nl blocks after
+// them: sum_i u_i (rhs_i - damping_i u_i) (Linearization::LinearDeltaError, linearization.h:62-67),
 // and in the same pass the two counts of the iteration's checks: entries of the damped diagonal
-// (undamped + damping) below eps in magnitude (CheckHessianDiagonal, lm.tcc:56-90) and
-// non-finite entries of the update (lm.tcc:225-227). Partials: part[b], part[nb + b],
-// part[2 nb + b].
-__global__ void __launch_bounds__(256) lde_partial_kernel(const double* __restrict__ u,
-                                                          const double* __restrict__ rhs,
-                                                          const double* __restrict__ damp,
-                                                          const double* __restrict__ und,
-                                                          double eps, int64_t n,
-                                                          double* __restrict__ part) {
+// (undamped + damping) below eps in magnitude (CheckHessianDiagonal, lm.tcc:56-90) and non-finite
+// entries of the update (lm.tcc:225-227), at part[kReduceBlocks], + nl and + 2 nl.
+__global__ void __launch_bounds__(256) lm_partials_kernel(
+    const double* __restrict__ residual, int64_t m, int nr, const double* __restrict__ u,
+    const double* __restrict__ rhs, const double* __restrict__ damp,
+    const double* __restrict__ und, double eps, int64_t n, int nl, double* __restrict__ part) {
   __shared__ double ws[3][4];
+  const int b = blockIdx.x;
   double acc = 0, zeros = 0, bad = 0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const double ui = u[i], di = damp[i];
-    acc += ui * (rhs[i] - di * ui);
-    zeros += fabs(und[i] + di) < eps ? 1.0 : 0.0;
-    bad += isfinite(ui) ? 0.0 : 1.0;
+  if (b < nr) {
+    for (int64_t i = b * (int64_t)256 + threadIdx.x; i < m; i += (int64_t)nr * 256)
+      acc += residual[i] * residual[i];
+  } else {
+    for (int64_t i = (b - nr) * (int64_t)256 + threadIdx.x; i < n; i += (int64_t)nl * 256) {
+      const double ui = u[i], di = damp[i];
+      acc += ui * (rhs[i] - di * ui);
+      zeros += fabs(und[i] + di) < eps ? 1.0 : 0.0;
+      bad += isfinite(ui) ? 0.0 : 1.0;
+    }
   }
   for (int o = 32; o > 0; o >>= 1) {
     acc += __shfl_down(acc, o, 64);
@@ -272,27 +255,87 @@ __global__ void __launch_bounds__(256) lde_partial_kernel(const double* __restri
     ws[2][threadIdx.x >> 6] = bad;
   }
   __syncthreads();
-  if (threadIdx.x < 3)
-    part[threadIdx.x * gridDim.x + blockIdx.x] =
-        ws[threadIdx.x][0] + ws[threadIdx.x][1] + ws[threadIdx.x][2] + ws[threadIdx.x][3];
+  if (threadIdx.x < 3) {
+    const double t = ws[threadIdx.x][0] + ws[threadIdx.x][1] + ws[threadIdx.x][2] +
+                     ws[threadIdx.x][3];
+    if (b >= nr) part[kReduceBlocks + threadIdx.x * nl + b - nr] = t;
+    else if (threadIdx.x == 0) part[b] = t;
+  }
 }
-__global__ void __launch_bounds__(256) sum_into_kernel(const double* __restrict__ part, int nb,
-                                                       double* __restrict__ out) {
-  __shared__ double ws[4];
+
+// Sum of part[0 .. nb) over a 256-thread block (valid in every thread).
+__device__ double block_total(const double* __restrict__ part, int nb, double* ws) {
   double acc = 0;
-  for (int i = threadIdx.x; i < nb; i += blockDim.x) acc += part[i];
+  for (int i = threadIdx.x; i < nb; i += 256) acc += part[i];
   for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
+  __syncthreads();  // the previous total has been read
   if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = acc;
   __syncthreads();
-  if (threadIdx.x == 0) *out = ws[0] + ws[1] + ws[2] + ws[3];
+  return ws[0] + ws[1] + ws[2] + ws[3];
+}
+
+// Second pass (one block) and what the host waits for. first >= 0: the error of that block and the
+// iteration -1 record (levenberg_marquardt_solver.tcc:158-186). Otherwise the sums of the step and
+// the accept / reject / lambda logic of Iterate (:239-340). The state goes to the host's pinned
+// mirror in the same kernel. Separate kernels for each sum, the decision and its copy cost a small
+// problem seven launches and a copy per iteration; without them, the copy of all Values and the
+// separate passes of the damping, a ten-pose smoothing run takes 1.06 ms (1.4 to 1.7 before) and a
+// 2503-node pose graph's 2.05 ms (2.25).
+__global__ void __launch_bounds__(256) lm_finish_kernel(LmDevState* st, LmDevState* mirror,
+                                                        const double* __restrict__ part, int nr,
+                                                        int nl, int first, int init, int nw,
+                                                        int best, int iteration,
+                                                        symhip_optimizer_params p,
+                                                        int have_last_update, double eps) {
+  __shared__ double ws[4];
+  const double err = 0.5 * block_total(part, nr, ws);
+  double lde = 0, zeros = 0, bad = 0;
+  if (first < 0) {
+    lde = block_total(part + kReduceBlocks, nl, ws);
+    zeros = block_total(part + kReduceBlocks + nl, nl, ws);
+    bad = block_total(part + kReduceBlocks + 2 * nl, nl, ws);
+  }
+  if (threadIdx.x != 0) return;
+  if (first >= 0) {
+    st->err[first] = err;
+    st->rec = symhip_iteration_stats{};
+    st->rec.iteration = -1;
+    st->rec.new_error = err;
+    st->rec.current_lambda = st->lambda;
+    st->status = isfinite(err) ? 0 : SYMHIP_STATUS_FAILED;
+    st->reason = isfinite(err) ? 0 : SYMHIP_FAILURE_INITIAL_ERROR_NOT_FINITE;
+  } else {
+    st->err[nw] = err;
+    st->lde = lde;
+    st->zero_diag = zeros;
+    st->nonfinite_update = bad;
+    const LmDecision d = lm_decide(st->err[init], err, st->err[best], lde, st->lambda, st->nu,
+                                   iteration, p, have_last_update, st->nl2, st->nu2, st->dotlu, eps);
+    st->rec = d.rec;
+    st->lambda = d.lambda;
+    st->nu = d.nu;
+    st->status = d.status;
+    st->reason = d.reason;
+    st->accept = d.accept;
+    st->set_best = d.set_best;
+  }
+  *mirror = *st;
+}
+
+// The error of a block alone (a stage's first linearization past the first record).
+__global__ void __launch_bounds__(256) lm_error_kernel(const double* __restrict__ part, int nr,
+                                                       double* __restrict__ out) {
+  __shared__ double ws[4];
+  const double err = 0.5 * block_total(part, nr, ws);
+  if (threadIdx.x == 0) *out = err;
 }
 
 // ---- CSC backend kernels ----
 __global__ void damp_csc_kernel(int32_t n, const int32_t* __restrict__ colptr,
-                                double* __restrict__ hval, const double* __restrict__ lambda_p,
-                                int use_diag, int keep_max, int have_max, double dmin, int unit,
-                                double* __restrict__ undamped, double* __restrict__ damping,
-                                double* __restrict__ max_diag) {
+                                const double* __restrict__ hval,
+                                const double* __restrict__ lambda_p, int use_diag, int keep_max,
+                                int have_max, double dmin, int unit, double* __restrict__ undamped,
+                                double* __restrict__ damping, double* __restrict__ max_diag) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
   const double lambda = *lambda_p;
@@ -310,12 +353,6 @@ __global__ void damp_csc_kernel(int32_t n, const int32_t* __restrict__ colptr,
   }
   if (unit) d += lambda;
   damping[j] = d;
-  hval[colptr[j]] = u + d;
-}
-__global__ void restore_csc_kernel(int32_t n, const int32_t* __restrict__ colptr,
-                                   double* __restrict__ hval, const double* __restrict__ undamped) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < n) hval[colptr[j]] = undamped[j];
 }
 __global__ void negate_kernel(int32_t n, const double* __restrict__ x, double* __restrict__ y) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -323,7 +360,7 @@ __global__ void negate_kernel(int32_t n, const double* __restrict__ x, double* _
 }
 
 // out = b - A x (b non-null) or out = A x, for the symmetric A held as its lower CSC (colptr,
-// rowind, vals): row i of A is column i's entries (rows >= i) and the entries (i, j), j < i,
+// rowind, vals) plus the damping on its diagonal: row i of A is column i's entries (rows >= i) and the entries (i, j), j < i,
 // which tptr / tcol / tidx list per row (column j and the entry's index in vals). One thread
 // per row, FP64, no atomics: the residuals and products of the mixed-precision form's
 // refinement.
@@ -331,11 +368,13 @@ __global__ void __launch_bounds__(256) sym_matvec_kernel(
     int32_t n, const int32_t* __restrict__ colptr, const int32_t* __restrict__ rowind,
     const double* __restrict__ vals, const int32_t* __restrict__ tptr,
     const int32_t* __restrict__ tcol, const int64_t* __restrict__ tidx,
-    const double* __restrict__ b, const double* __restrict__ x, double* __restrict__ out) {
+    const double* __restrict__ damping, const double* __restrict__ b, const double* __restrict__ x,
+    double* __restrict__ out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  double acc = 0.0;
-  for (int32_t e = colptr[i]; e < colptr[i + 1]; ++e) acc += vals[e] * x[rowind[e]];
+  const int32_t d = colptr[i];  // the diagonal entry comes first
+  double acc = (vals[d] + damping[i]) * x[i];
+  for (int32_t e = d + 1; e < colptr[i + 1]; ++e) acc += vals[e] * x[rowind[e]];
   for (int32_t e = tptr[i]; e < tptr[i + 1]; ++e) acc += vals[tidx[e]] * x[tcol[e]];
   out[i] = b ? b[i] - acc : acc;
 }
@@ -399,9 +438,8 @@ class CscBackend final : public SystemBackend {
   ~CscBackend() override {
     if (host_sums_) (void)hipHostFree(host_sums_);
   }
-  void relinearize(int b, const double* values, double* err_out, hipStream_t s) override {
+  void relinearize(int b, const double* values, hipStream_t s) override {
     lin_.run(values, residual_[b].get(), hval_[b].get(), rhs_[b].get(), s);
-    half_squared_norm(residual_[b].get(), M_, partials_.get(), err_out, s);
   }
   void damp(int b, const double* lambda_dev, const symhip_optimizer_params& p,
             bool have_max_diagonal, hipStream_t s) override {
@@ -411,19 +449,19 @@ class CscBackend final : public SystemBackend {
                        p.diagonal_damping_min, p.use_unit_damping, undamped_.get(),
                        damping_.get(), max_diag_.get());
   }
-  void restore(int b, hipStream_t s) override {
-    hipLaunchKernelGGL(restore_csc_kernel, dim3(grid_for(N_, 256)), dim3(256), 0, s, N_,
-                       colptr_.get(), hval_[b].get(), undamped_.get());
-  }
   void solve(int b, double* update, hipStream_t s) override {
     {
       PhaseScope ps(timer_, SYMHIP_PHASE_FACTOR, s);
       // the forward solve runs inside the factorization
-      chol_.factorize(hval_[b].get(), s, rhs_[b].get());
+      chol_.factorize(hval_[b].get(), s, rhs_[b].get(), damping_.get());
     }
     PhaseScope ps(timer_, SYMHIP_PHASE_SOLVE, s);
+    if (!chol_.f32_updates()) {
+      chol_.solve_fused(update, s, /*negate=*/true);
+      return;
+    }
     chol_.solve_fused(x_.get(), s);
-    if (chol_.f32_updates()) refine(b, s);
+    refine(b, s);
     hipLaunchKernelGGL(negate_kernel, dim3(grid_for(N_, 256)), dim3(256), 0, s, N_, x_.get(),
                        update);
   }
@@ -493,7 +531,8 @@ class CscBackend final : public SystemBackend {
     double* sc = sums_.get();  // 0: b.b, 1: r.r, 2: p.q, 3 + (k & 1): r.z of iteration k
     auto matvec = [&](const double* rhs, const double* v, double* out) {
       hipLaunchKernelGGL(sym_matvec_kernel, g, blk, 0, s, N_, colptr_.get(), rowind_.get(),
-                         hval_[b].get(), tptr_.get(), tcol_.get(), tidx_.get(), rhs, v, out);
+                         hval_[b].get(), tptr_.get(), tcol_.get(), tidx_.get(), damping_.get(),
+                         rhs, v, out);
     };
     auto read = [&]() {
       HIP_OK(hipMemcpyAsync(host_sums_, sc, 5 * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -544,7 +583,7 @@ class CscBackend final : public SystemBackend {
     }
     if (!ok) {
       chol_.set_f32_updates(false);
-      chol_.factorize(hval_[b].get(), s, rhs_[b].get());
+      chol_.factorize(hval_[b].get(), s, rhs_[b].get(), damping_.get());
       chol_.solve_fused(x, s);
       chol_.set_f32_updates(true);
       matvec(rhs_[b].get(), x, r);
@@ -641,7 +680,7 @@ DeviceOptimizer::DeviceOptimizer(const symhip_problem_desc* d, const symhip_opti
   for (auto& v : values_) v.resize(std::max<int64_t>(1, host_.storage_total));
   update_.resize(std::max(1, host_.N));
   last_update_.resize(std::max(1, host_.N));
-  partials_.resize(3 * kReduceBlocks);
+  partials_.resize(4 * kReduceBlocks);
   std::vector<int32_t> rt, rs, rto;
   for (int32_t k : host_.state_keys) {
     rt.push_back(host_.types[k]);
@@ -687,7 +726,7 @@ void DeviceOptimizer::best_linearization(double* residual, double* hval, double*
 void DeviceOptimizer::relinearize(int b) {
   {
     PhaseScope ps(&timer_, SYMHIP_PHASE_LINEARIZE, stream_);
-    backend_->relinearize(b, values_[b].get(), &dstate_->err[b], stream_);
+    backend_->relinearize(b, values_[b].get(), stream_);
   }
   linearized_[b] = true;
   if (p_.include_jacobians) fill_jacobian(b);
@@ -902,7 +941,7 @@ void DeviceOptimizer::reset_run() {
   have_last_update_ = false;
   for (int b = 0; b < 3; ++b) linearized_[b] = false;
   valid_[new_] = true;
-  valid_[init_] = valid_[free_] = false;
+  valid_[init_] = valid_[free_] = false;  // their constants are last run's
   hipLaunchKernelGGL(lm_reset_kernel, dim3(1), dim3(1), 0, stream_, dstate_, p_.initial_lambda,
                      p_.dynamic_lambda_update_beta);
   backend_->begin_run();
@@ -1038,6 +1077,8 @@ bool DeviceOptimizer::iterate(std::vector<symhip_iteration_stats>& iters, int32_
                               int& status, int& reason) {
   std::swap(init_, new_);  // state_.Step()
   iteration_++;
+  // first pass blocks of the reductions
+  const int nr = std::max(1, std::min(kReduceBlocks, grid_for(host_.M, 256)));
   if (!linearized_[init_]) {
     relinearize(init_);
     // SetBestToInit
@@ -1045,10 +1086,17 @@ bool DeviceOptimizer::iterate(std::vector<symhip_iteration_stats>& iters, int32_
       if (best_ != new_) free_ = best_;
       best_ = init_;
     }
+    hipLaunchKernelGGL(lm_partials_kernel, dim3(nr), dim3(256), 0, stream_,
+                       backend_->residual(init_), (int64_t)host_.M, nr, nullptr, nullptr, nullptr,
+                       nullptr, 0.0, (int64_t)0, 0, partials_.get());
+    if (iteration_ > 0)
+      hipLaunchKernelGGL(lm_error_kernel, dim3(1), dim3(256), 0, stream_, partials_.get(), nr,
+                         &dstate_->err[init_]);
   }
   if (iteration_ == 0) {
-    hipLaunchKernelGGL(lm_first_record_kernel, dim3(1), dim3(1), 0, stream_, dstate_, init_);
-    HIP_OK(hipMemcpyAsync(hstate_, dstate_, sizeof(LmDevState), hipMemcpyDeviceToHost, stream_));
+    hipLaunchKernelGGL(lm_finish_kernel, dim3(1), dim3(256), 0, stream_, dstate_, hstate_,
+                       partials_.get(), nr, 0, init_, init_, new_, best_, iteration_, p_, 0,
+                       epsilon_);
     HIP_OK(hipStreamSynchronize(stream_));
     iters.push_back(hstate_->rec);
     if (p_.debug_stats) record_debug(init_, false);
@@ -1071,47 +1119,43 @@ bool DeviceOptimizer::iterate(std::vector<symhip_iteration_stats>& iters, int32_
   }
   if (p_.use_diagonal_damping && p_.keep_max_diagonal_damping) have_max_diagonal_ = true;
   backend_->solve(init_, update_.get(), stream_);
-  backend_->restore(init_, stream_);
-  // UpdateNewFromInit: copy Init values into New, then retract the optimized keys.
+  // UpdateNewFromInit: the optimized keys retracted from Init into New. The other keys are
+  // constants: a block gets them with its first use in a run.
   {
     PhaseScope ps(&timer_, SYMHIP_PHASE_RETRACT, stream_);
-    HIP_OK(hipMemcpyAsync(values_[new_].get(), values_[init_].get(),
-                          sizeof(double) * host_.storage_total, hipMemcpyDeviceToDevice,
-                          stream_));
+    if (!valid_[new_])
+      HIP_OK(hipMemcpyAsync(values_[new_].get(), values_[init_].get(),
+                            sizeof(double) * host_.storage_total, hipMemcpyDeviceToDevice,
+                            stream_));
     valid_[new_] = true;
     const int32_t nk = (int32_t)host_.state_keys.size();
     hipLaunchKernelGGL(retract_kernel, dim3(grid_for(nk, 256)), dim3(256), 0, stream_, nk,
                        retract_type_.get(), retract_soff_.get(), retract_toff_.get(),
-                       update_.get(), values_[new_].get(), epsilon_);
+                       update_.get(), values_[init_].get(), values_[new_].get(), epsilon_);
   }
   relinearize(new_);
   const int decide_ev = timer_.begin(SYMHIP_PHASE_DECIDE, stream_);
-  {
-    const int nb = std::max(1, std::min(kReduceBlocks, grid_for(N, 256)));
-    hipLaunchKernelGGL(lde_partial_kernel, dim3(nb), dim3(256), 0, stream_, update_.get(),
-                       backend_->rhs(init_), backend_->damping(), backend_->undamped_diagonal(),
-                       epsilon_, (int64_t)N, partials_.get());
-    hipLaunchKernelGGL(sum_into_kernel, dim3(1), dim3(256), 0, stream_, partials_.get(), nb,
-                       &dstate_->lde);
-    hipLaunchKernelGGL(sum_into_kernel, dim3(1), dim3(256), 0, stream_, partials_.get() + nb, nb,
-                       &dstate_->zero_diag);
-    hipLaunchKernelGGL(sum_into_kernel, dim3(1), dim3(256), 0, stream_,
-                       partials_.get() + 2 * nb, nb, &dstate_->nonfinite_update);
-  }
+  const int nl = std::max(1, std::min(kReduceBlocks, grid_for(N, 256)));
+  hipLaunchKernelGGL(lm_partials_kernel, dim3(nr + nl), dim3(256), 0, stream_,
+                     backend_->residual(new_), (int64_t)host_.M, nr, update_.get(),
+                     backend_->rhs(init_), backend_->damping(), backend_->undamped_diagonal(),
+                     epsilon_, (int64_t)N, nl, partials_.get());
   if (p_.enable_bold_updates && have_last_update_) {
-    dot(last_update_.get(), last_update_.get(), N, partials_.get(), &dstate_->nl2, stream_);
-    dot(update_.get(), update_.get(), N, partials_.get(), &dstate_->nu2, stream_);
-    dot(last_update_.get(), update_.get(), N, partials_.get(), &dstate_->dotlu, stream_);
+    bold_partials_.resize(kReduceBlocks);
+    double* part = bold_partials_.get();
+    dot(last_update_.get(), last_update_.get(), N, part, &dstate_->nl2, stream_);
+    dot(update_.get(), update_.get(), N, part, &dstate_->nu2, stream_);
+    dot(last_update_.get(), update_.get(), N, part, &dstate_->dotlu, stream_);
   }
   // An inexact (truncated PCG) step whose reduction falls below the early-exit threshold switches
   // the solver to exact steps instead of ending the run; the early exit applies to those.
   symhip_optimizer_params pd = p_;
   const bool deferred = backend_->defers_early_exit();
   if (deferred) pd.early_exit_min_reduction = 0.0;
-  hipLaunchKernelGGL(lm_decide_kernel, dim3(1), dim3(1), 0, stream_, dstate_, init_, new_, best_,
-                     iteration_, pd, have_last_update_ ? 1 : 0, epsilon_);
+  hipLaunchKernelGGL(lm_finish_kernel, dim3(1), dim3(256), 0, stream_, dstate_, hstate_,
+                     partials_.get(), nr, nl, -1, init_, new_, best_, iteration_, pd,
+                     have_last_update_ ? 1 : 0, epsilon_);
   timer_.end(decide_ev, stream_);
-  HIP_OK(hipMemcpyAsync(hstate_, dstate_, sizeof(LmDevState), hipMemcpyDeviceToHost, stream_));
   HIP_OK(hipStreamSynchronize(stream_));
   timer_.collect();
   HIP_OK(hipGetLastError());
@@ -1133,8 +1177,9 @@ bool DeviceOptimizer::iterate(std::vector<symhip_iteration_stats>& iters, int32_
     std::swap(new_, init_);  // SwapNewAndInit
   } else {
     have_last_update_ = true;
-    HIP_OK(hipMemcpyAsync(last_update_.get(), update_.get(), sizeof(double) * N,
-                          hipMemcpyDeviceToDevice, stream_));
+    if (p_.enable_bold_updates)  // read by the bold-update test alone
+      HIP_OK(hipMemcpyAsync(last_update_.get(), update_.get(), sizeof(double) * N,
+                            hipMemcpyDeviceToDevice, stream_));
     if (hstate_->set_best) {
       // SetBestToNew
       if (best_ != new_) {

@@ -802,10 +802,9 @@ __global__ void scatter_kernel(int32_t n, const int32_t* __restrict__ idx,
 class SchurBackend final : public SystemBackend {
  public:
   SchurBackend(const HostProblem& p, const SolverOptions& o, hipStream_t s);
-  void relinearize(int b, const double* values, double* err_out, hipStream_t s) override;
+  void relinearize(int b, const double* values, hipStream_t s) override;
   void damp(int b, const double* lambda_dev, const symhip_optimizer_params& p,
             bool have_max_diagonal, hipStream_t s) override;
-  void restore(int, hipStream_t) override {}  // damping is applied out of place
   void solve(int b, double* update, hipStream_t s) override;
   const double* rhs(int b) const override { return rhs_[b].get(); }
   const double* residual(int b) const override { return residual_[b].get(); }
@@ -886,8 +885,7 @@ class SchurBackend final : public SystemBackend {
   std::vector<BGroup> bgroups_;
   // per state block storage
   DBuf<double> residual_[3], W_[3], V_[3], gp_[3], Bdiag_[3], Bfac_[3], gB_[3], rhs_[3];
-  DBuf<double> damping_, undamped_, max_diag_, dnode_, dpoint_, Lp_, hp_, Z_, ZZ_, v_, y_,
-      partials_;
+  DBuf<double> damping_, undamped_, max_diag_, dnode_, dpoint_, Lp_, hp_, Z_, ZZ_, v_, y_;
   // FP32 form (precision 1): while PCG runs, W and Z are stored in FP32 (W32_, Z32_) and so is S
   // for PCG; residual, gradient, sums, LDL^T and the LM decisions stay FP64. Once the run has
   // switched to the exact LDL^T (exact_now_), linearization returns to plain FP64 storage, the
@@ -1255,7 +1253,7 @@ SchurBackend::SchurBackend(const HostProblem& P, const SolverOptions& o, hipStre
     pld[k] = ld;
     ptrans[k] = trans ? 1 : 0;
   }
-  chol_.setup(sym, scp.data(), sri.data(), s);
+  chol_.setup(sym, nullptr, nullptr, s);
   if (o.use_pcg) {
     SYMHIP_CHECK(o.pcg_max_iters >= 1 && o.pcg_rel_tol > 0 && o.pcg_rel_tol < 1,
                  "PCG needs pcg_max_iters >= 1 and 0 < pcg_rel_tol < 1");
@@ -1394,7 +1392,6 @@ SchurBackend::SchurBackend(const HostProblem& P, const SolverOptions& o, hipStre
   ZZ_.resize((size_t)n_nodes_ * nde);
   v_.resize((size_t)n_nodes_ * nd_);
   y_.resize((size_t)n_nodes_ * nd_);
-  partials_.resize(kReduceBlocks);
   HIP_OK(hipStreamSynchronize(s));
 }
 
@@ -1437,9 +1434,8 @@ void SchurBackend::relin_nd(int b, const double* values, hipStream_t s) {
   HIP_OK(hipGetLastError());
 }
 
-void SchurBackend::relinearize(int b, const double* values, double* err_out, hipStream_t s) {
+void SchurBackend::relinearize(int b, const double* values, hipStream_t s) {
   if (nd_ == 9) relin_nd<9>(b, values, s); else relin_nd<6>(b, values, s);
-  half_squared_norm(residual_[b].get(), M_, partials_.get(), err_out, s);
 }
 
 void SchurBackend::damp(int b, const double* lambda_dev, const symhip_optimizer_params& p,

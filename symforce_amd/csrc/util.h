@@ -14,10 +14,7 @@ void fill_zero(double* p, int64_t n, hipStream_t s);
 void fill_zero(float* p, int64_t n, hipStream_t s);
 void fill_zero_i32(int32_t* p, int64_t n, hipStream_t s);
 
-// Deterministic two-pass FP64 reductions into a device scalar (out[0]).
-// sum_sq: out = 0.5 * sum(x^2)  (Linearization::Error, opt/linearization.h:51-54)
-void half_squared_norm(const double* x, int64_t n, double* partials, double* out, hipStream_t s);
-// out = sum(a .* b)
+// Deterministic two-pass FP64 reduction into a device scalar: out[0] = sum(a .* b).
 void dot(const double* a, const double* b, int64_t n, double* partials, double* out, hipStream_t s);
 constexpr int kReduceBlocks = 1024;
 

@@ -27,16 +27,6 @@ __device__ double block_sum(double v) {
   return t;
 }
 
-__global__ void __launch_bounds__(256) sq_partial_kernel(const double* __restrict__ x, int64_t n,
-                                                         double* __restrict__ partials) {
-  double acc = 0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    acc += x[i] * x[i];
-  acc = block_sum(acc);
-  if (threadIdx.x == 0) partials[blockIdx.x] = acc;
-}
-
 __global__ void __launch_bounds__(256) dot_partial_kernel(const double* __restrict__ a,
                                                           const double* __restrict__ b, int64_t n,
                                                           double* __restrict__ partials) {
@@ -49,11 +39,11 @@ __global__ void __launch_bounds__(256) dot_partial_kernel(const double* __restri
 }
 
 __global__ void __launch_bounds__(256) finish_kernel(const double* __restrict__ partials, int nb,
-                                                     double scale, double* __restrict__ out) {
+                                                     double* __restrict__ out) {
   double acc = 0;
   for (int i = threadIdx.x; i < nb; i += blockDim.x) acc += partials[i];
   acc = block_sum(acc);
-  if (threadIdx.x == 0) out[0] = scale * acc;
+  if (threadIdx.x == 0) out[0] = acc;
 }
 
 }  // namespace
@@ -77,18 +67,11 @@ void fill_zero_i32(int32_t* p, int64_t n, hipStream_t s) {
   HIP_OK(hipGetLastError());
 }
 
-void half_squared_norm(const double* x, int64_t n, double* partials, double* out, hipStream_t s) {
-  const int nb = (int)std::max<int64_t>(1, std::min<int64_t>(kReduceBlocks, grid_for(n, 256)));
-  hipLaunchKernelGGL(sq_partial_kernel, dim3(nb), dim3(256), 0, s, x, n, partials);
-  hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(256), 0, s, partials, nb, 0.5, out);
-  HIP_OK(hipGetLastError());
-}
-
 void dot(const double* a, const double* b, int64_t n, double* partials, double* out,
          hipStream_t s) {
   const int nb = (int)std::max<int64_t>(1, std::min<int64_t>(kReduceBlocks, grid_for(n, 256)));
   hipLaunchKernelGGL(dot_partial_kernel, dim3(nb), dim3(256), 0, s, a, b, n, partials);
-  hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(256), 0, s, partials, nb, 1.0, out);
+  hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(256), 0, s, partials, nb, out);
   HIP_OK(hipGetLastError());
 }
 
