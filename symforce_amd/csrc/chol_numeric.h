@@ -87,16 +87,19 @@ class SupernodalLDLT {
   bool f32_updates_ = false;
   CholSymbolic sym_;
   DBuf<double> panel_, l11_, D_, y_, yout_, part_;
+  DBuf<unsigned long long> ysol_;  // the backward launch's results as its blocks see them
+  DBuf<int32_t> ticket_;
   DBuf<int32_t> counter_;  // per-supernode arrival counters of the backward pass (self-resetting)
   DBuf<double> many_y_, many_yout_, many_part_;  // solve_many
   DBuf<int32_t> many_counter_;                   // per (right-hand-side group, supernode)
   DBuf<int64_t> scat_col_;
   DBuf<int32_t> panel_src_, diag_pos_;  // factorize(): what each panel entry is assembled from
   DBuf<int32_t> rows_, perm_, upd_rel_, scat_rel_;
-  DBuf<uint8_t> trsm_tasks_, upd_tasks_, solve_tasks_;  // per-level task lists (chol_numeric.hip)
+  DBuf<uint8_t> trsm_tasks_, upd_tasks_, solve_tasks_, chain_tasks_;  // per-level task lists (chol_numeric.hip)
   // work lists (flattened over levels)
   std::vector<int32_t> lvl_snode_ptr_, lvl_trsm_ptr_, lvl_upd_ptr_, lvl_solve_ptr_;
   DBuf<int32_t> lvl_snodes_;
+  int32_t chain_levels_ = 0, n_chain_ = 0;  // levels and tasks of the backward launch
 };
 
 }  // namespace symhip
