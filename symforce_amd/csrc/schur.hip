@@ -398,7 +398,7 @@ __global__ void __launch_bounds__(256) point_elim_kernel(int32_t n_obs,
 // One wavefront per S block (a, b): S = [Bdiag + damping - ZZ_a if a == b] + Bfac
 // - sum_pairs Z_x Z_y^T. The pair sum is the product X Y^T with X = [Z_x1 Z_x2 ...] (ND x 3P)
 // and Y = [Z_y1 Z_y2 ...], so K = 3P is packed densely into FP64 matrix-core steps
-// (v_mfma_f64_16x16x4f64; a batch of four pairs = 12 K entries = three MFMAs): at step h lane l
+// (v_mfma_f64_16x16x4f64; a batch of eight pairs = 24 K entries = six MFMAs): at step h lane l
 // feeds A(i = l % 16, k = l / 16) = X(i, 4h + k) and B(k, j = l % 16) = Y(j, 4h + k) (rows
 // i >= ND and K entries past the block's pairs are zero) and holds D(l / 16 + 4 r, l % 16) in
 // accumulator register r (the FP64 16x16x4 output interleaves rows across the four lane groups).
@@ -416,7 +416,7 @@ __global__ void __launch_bounds__(256) point_elim_kernel(int32_t n_obs,
 // (transposed). Z is read as TW (FP32 in the FP32 form) and widened: the sums are FP64 on the
 // matrix cores either way; the full storage is written as TS.
 constexpr int kRcsChunk = 512;  // pairs per work item at most
-constexpr int kRcsBatch = 4;    // pairs per batch (a multiple of 4: 3 K entries per pair, 4 per MFMA)
+constexpr int kRcsBatch = 8;    // pairs per batch (a multiple of 4: 3 K entries per pair, 4 per MFMA)
 constexpr bool kRcsHeaviestFirst = false;  // order each XCD's items by size (else by camera row)
 constexpr double kRcsTailFrac = 0.4;       // row order: share of the pairs dealt heaviest first
 constexpr int kRcsTailChunk = 256;         // row order: pairs per item at most in that tail
@@ -480,11 +480,15 @@ __global__ void __launch_bounds__(256) rcs_assemble_kernel(
   // loads are always issued (a batch past the item's end re-reads its first pairs) to keep the
   // wait count fixed.
   auto fetch_idx = [&](int qb, int (&ix)[NI]) {
-    const int qs = qb < q_end ? qb : q_begin;
+    int qs = qb < q_end ? qb : q_begin;
+    asm volatile("" : "+s"(qs)::"memory");  // not before the copies issued so far
 #pragma unroll
     for (int u = 0; u < NI; ++u) ix[u] = pairs[2 * qs + slot_o[u]];
   };
-  auto issue = [&](const int (&ix)[NI], char* buf) {
+  auto issue = [&](int (&ix)[NI], char* buf) {
+    // every index is waited for before the first copy: a wait after it would wait for the copy too
+#pragma unroll
+    for (int u = 0; u < NI; ++u) asm volatile("" : "+v"(ix[u])::"memory");
 #pragma unroll
     for (int u = 0; u < NI; ++u) {
       const char* src = reinterpret_cast<const char*>(Z + (int64_t)ix[u] * ZS) + slot_c[u] * 16;
@@ -540,17 +544,20 @@ __global__ void __launch_bounds__(256) rcs_assemble_kernel(
       }
     }
   };
-  auto consume = [&](int q, const char* buf) {
+  // Only the item's last batch masks pairs past its end. Rows i >= ND (read as row 0) need no mask:
+  // they reach output rows and columns >= ND only, which are not stored.
+  auto consume = [&]<bool kTail>(int q, const char* buf) {
     const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)buf;
     double av[NH], bv[NH];
 #pragma unroll
     for (int g = 0; g < NH; g += 3) read3(base, g, av + g, bv + g);
+    if constexpr (kTail) {
 #pragma unroll
-    for (int h = 0; h < NH; ++h) {
-      const int p = (4 * h + kg) / 3;
-      const bool ok = live && q + p < q_end;
-      av[h] = ok ? av[h] : 0.0;
-      bv[h] = ok ? bv[h] : 0.0;
+      for (int h = 0; h < NH; ++h) {
+        const bool ok = q + (4 * h + kg) / 3 < q_end;
+        av[h] = ok ? av[h] : 0.0;
+        bv[h] = ok ? bv[h] : 0.0;
+      }
     }
 #pragma unroll
     for (int h = 0; h < NH; ++h)
@@ -559,15 +566,25 @@ __global__ void __launch_bounds__(256) rcs_assemble_kernel(
   // Per batch: copy batch k, fetch batch k + 1's indices, wait for the copy (the index loads
   // issued after it may stay in flight: vector memory operations complete in order), read,
   // multiply. (A second buffer, batch k + 1's copy overlapping batch k's reads and products,
-  // measured no faster: the launch is bound by the copies' HBM and L2 traffic, not by a wave's
-  // latency.)
+  // measured no faster.) Batches of eight pairs, all copies of one issued together and no masks
+  // outside the last: with four, a wait for the second copy's index after the first copy's issue
+  // and the masks the launch was bound by its waves, in FP32 too: 232 -> 192 us in FP32 at 1000
+  // cameras with 200 000 points, 44 -> 33 us in FP64 at 137 cameras with 9001; in FP64 at 1000
+  // cameras it stays at 240 us, bound by the copies' traffic.
   int ix[NI];
   fetch_idx(q_begin, ix);
-  for (int q = q_begin; q < q_end; q += NB) {
+  int q = q_begin;
+  for (; q + NB <= q_end; q += NB) {
     issue(ix, lds_z[w]);
     fetch_idx(q + NB, ix);
+    __builtin_amdgcn_sched_barrier(0);  // the index loads stay after the copies, before the wait
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NI) : "memory");
-    consume(q, lds_z[w]);
+    consume.template operator()<false>(q, lds_z[w]);
+  }
+  if (q < q_end) {
+    issue(ix, lds_z[w]);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    consume.template operator()<true>(q, lds_z[w]);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last index loads
   const d4 sum = acc;
