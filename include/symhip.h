@@ -91,10 +91,10 @@ int symhip_batch_solve(symhip_batch_t batch, double* values_out,
 /* Autotuner of the batched solve (no counterpart in the reference): solves the whole batch
    `reps` times in each of the 4 launch configurations (bit 0: the kernel built for two
    wavefronts per SIMD instead of one, i.e. as many more resident problems as their shared memory
-   leaves room for, at ~110 spilled registers; bit 1: problems with the most poses launched first) and keeps the fastest for
-   later symhip_batch_solve calls. config_ms (4 entries, may be NULL) receives each one's best
-   launch time, *chosen (may be NULL) the configuration kept. The results of every
-   configuration are the same. */
+   leaves room for, at ~110 spilled registers; bit 1: problems with the most poses launched first)
+   and keeps the fastest for later symhip_batch_solve calls. config_ms (4 entries, may be NULL)
+   receives each one's best launch time, *chosen (may be NULL) the configuration kept. The results
+   of every configuration are the same. */
 int symhip_batch_tune(symhip_batch_t batch, int32_t reps, double* config_ms, int32_t* chosen);
 /* Selects launch configuration `config` (0-3, as above) for later solves, e.g. one a previous
    tuning run of the same batch shape chose. */

@@ -497,15 +497,14 @@ void chol_symbolic(int32_t n, const int32_t* colptr, const int32_t* rowind,
   }
 }
 
-void chol_panel_sources(const CholSymbolic& s, const int32_t* colptr, const int32_t* rowind,
-                        std::vector<int32_t>& src, std::vector<int32_t>& diag) {
+std::vector<int64_t> chol_assembly_map(const CholSymbolic& s, const int32_t* colptr,
+                                       const int32_t* rowind) {
   const int32_t n = s.n;
   // supernode of each permuted column
   std::vector<int32_t> sn_of_col(n);
   for (int32_t k = 0; k < s.n_snodes; ++k)
     for (int32_t c = s.sn_col_begin[k]; c < s.sn_col_begin[k + 1]; ++c) sn_of_col[c] = k;
-  src.assign(s.panel_size(), kPanelFill);
-  diag.assign(n, 0);
+  std::vector<int64_t> map(colptr[n]);
   for (int32_t c = 0; c < n; ++c)
     for (int32_t q = colptr[c]; q < colptr[c + 1]; ++q) {
       int32_t pr = s.perm[rowind[q]], pc = s.perm[c];
@@ -523,10 +522,9 @@ void chol_panel_sources(const CholSymbolic& s, const int32_t* colptr, const int3
         rp = (int32_t)(it - (s.sn_rows.data() + s.sn_rows_ptr[t]));
       }
       const int64_t ld = s.sn_rows_ptr[t + 1] - s.sn_rows_ptr[t];
-      const bool on_diag = rowind[q] == c;
-      src[s.sn_panel_off[t] + (int64_t)(pc - c0) * ld + rp] = on_diag ? -2 - c : q;
-      if (on_diag) diag[c] = q;
+      map[q] = s.sn_panel_off[t] + (int64_t)(pc - c0) * ld + rp;
     }
+  return map;
 }
 
 }  // namespace symhip

@@ -74,11 +74,9 @@ void chol_symbolic(int32_t n, const int32_t* colptr, const int32_t* rowind,
                    const std::vector<int32_t>* given_node_order, int32_t max_cols,
                    CholSymbolic& out);
 
-// What each entry of the panel storage is assembled from: q >= 0 is entry q of the lower CSC input
-// matrix, -2 - j its diagonal entry of column j (at diag[j]), kPanelFill neither (fill-in, zero).
-constexpr int32_t kPanelFill = -1;
-void chol_panel_sources(const CholSymbolic& s, const int32_t* colptr, const int32_t* rowind,
-                        std::vector<int32_t>& src, std::vector<int32_t>& diag);
+// For each lower-pattern entry q of the input matrix, its position in the panel storage.
+std::vector<int64_t> chol_assembly_map(const CholSymbolic& s, const int32_t* colptr,
+                                       const int32_t* rowind);
 
 // Reference-convention elimination tree parent and column counts of the scalar factor for the
 // permuted pattern (sparse_cholesky_solver.tcc:55-89), used to check the symbolic layer.
