@@ -147,12 +147,14 @@ __device__ __forceinline__ double linearize(const BatchView& v, int b, int g0, i
   // lane + 32 (lane + 16, ..), which take its factors in turn. A lane takes kMatch of them at a
   // time: their offsets in one round of loads, their inputs in the next (one factor after the
   // other waits for both rounds; the compiler sinks a hand-pipelined loop's loads back to their
-  // uses). Past the list's end the last factor repeats with an infinite sigma, which adds zeros.
+  // uses). Past the list's end the last factor repeats with an infinite sigma, which adds zeros. A
+  // problem without poses (hand-made tables) reads row g0 in place of a row before the tables: an
+  // entry of match_ptr in any case, and of the pose blocks or the linearizations behind them.
   {
     constexpr int kMatch = 4;
     const int stride = n <= 16 ? 16 : n <= 32 ? 32 : 64;
     const int parts = 64 / stride, i = lane & (stride - 1), part = lane / stride;
-    const int gm = g0 + min(i, n - 1);
+    const int gm = g0 + min(i, max(n, 1) - 1);
     const double* pose = v.vals + (b * TP + gm) * 7;
     const int m0 = v.match_ptr[gm], m1 = i < n ? v.match_ptr[gm + 1] : m0;
     double p[7];

@@ -52,8 +52,14 @@ def hip():
     return _Hip()
 
 
-def _solve_noalloc(hip, probs, params, precision):
+def _solve_noalloc(hip, probs, params, precision, empty=()):
+    """empty: places in the batch that get a problem without poses (and without an entry of probs)."""
     t = capi.batch_pack(probs, params)
+    probs = list(probs)
+    for i in sorted(empty):
+        probs.insert(i, None)
+        t["pose_begin"] = np.insert(t["pose_begin"], i, t["pose_begin"][i])
+        t["n_problems"] += 1
     names = ("pose_begin", "pose_soff", "match_ptr", "match_args", "odo_args", "values")
     dev = {k: hip.upload(t[k]) for k in names}
     n, stride = len(probs), params.iterations + 1
@@ -80,10 +86,11 @@ def _solve_noalloc(hip, probs, params, precision):
         st = stats[i]
         sub = (capi.IterationStats * stride).from_address(C.addressof(iters) +
                                                           i * stride * sz_iter)
-        out.append(dict(values=values[off:off + len(prob.values)].copy(), status=st.status,
+        size = 0 if prob is None else len(prob.values)
+        out.append(dict(values=values[off:off + size].copy(), status=st.status,
                         failure_reason=st.failure_reason, best_index=st.best_index,
                         iterations=capi.iteration_records(sub, st.num_iterations)))
-        off += len(prob.values)
+        off += size
     return out
 
 
@@ -107,6 +114,22 @@ def test_noalloc_matches_batch_solve_on_two_calls(hip, precision):
         got = _solve_noalloc(hip, probs, params, precision)
         _assert_identical(got, want)
         assert all(r["status"] == capi.STATUS_SUCCESS for r in got)
+
+
+@pytest.mark.parametrize("precision", [capi.PRECISION_F64, capi.PRECISION_F32_JAC])
+def test_noalloc_problems_without_poses(hip, precision):
+    """Tables with empty problems before, between and after the others: nothing is read for them
+    (the first one's rows would lie before the tables, the last one's behind them), they end at
+    once with a zero error, and the others' results do not change."""
+    params = capi.default_params(iterations=30)
+    probs = capi.gen_localization_batch(5, seed=34)
+    want = _solve_noalloc(hip, probs, params, precision)
+    at = (0, 3, 7)
+    got = _solve_noalloc(hip, probs, params, precision, empty=at)
+    _assert_identical([r for i, r in enumerate(got) if i not in at], want)
+    for i in at:
+        assert got[i]["status"] == capi.STATUS_SUCCESS
+        assert [it["new_error"] for it in got[i]["iterations"]] == [0.0, 0.0]
 
 
 def test_noalloc_rejects_batches_beyond_the_scratch_size(hip):
