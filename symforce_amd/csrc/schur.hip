@@ -476,14 +476,20 @@ __global__ void __launch_bounds__(256) rcs_assemble_kernel(
     slot_c[u] = sl < SLOTS ? sl % CPO : 0;
   }
   // Each lane fetches the observation index of its own slots with vector loads, one batch
-  // ahead (after the batch's copy, so the wait for the copy leaves them in flight). The index
-  // loads are always issued (a batch past the item's end re-reads its first pairs) to keep the
-  // wait count fixed.
+  // ahead (after the batch's copy, so the wait for the copy leaves them in flight). That wait
+  // counts on exactly these NI loads behind the copies: they are always issued (a batch past the
+  // item's end re-reads its first pairs), and as relaxed atomic loads, plain loads in the machine
+  // code, the compiler neither drops them where their values are not used nor moves them over the
+  // copies or the wait. (Waiting for everything, with the index loads ahead of the copies, needs no
+  // count and is slower: 257 us against 230 in FP64 at 1000 cameras, 35 against 33 at 137.)
   auto fetch_idx = [&](int qb, int (&ix)[NI]) {
     int qs = qb < q_end ? qb : q_begin;
     asm volatile("" : "+s"(qs)::"memory");  // not before the copies issued so far
 #pragma unroll
-    for (int u = 0; u < NI; ++u) ix[u] = pairs[2 * qs + slot_o[u]];
+    for (int u = 0; u < NI; ++u)
+      ix[u] = __hip_atomic_load(pairs + 2 * qs + slot_o[u], __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_WAVEFRONT);
+    asm volatile("" ::: "memory");
   };
   auto issue = [&](int (&ix)[NI], char* buf) {
     // every index is waited for before the first copy: a wait after it would wait for the copy too
@@ -568,9 +574,9 @@ __global__ void __launch_bounds__(256) rcs_assemble_kernel(
   // multiply. (A second buffer, batch k + 1's copy overlapping batch k's reads and products,
   // measured no faster.) Batches of eight pairs, all copies of one issued together and no masks
   // outside the last: with four, a wait for the second copy's index after the first copy's issue
-  // and the masks the launch was bound by its waves, in FP32 too: 232 -> 192 us in FP32 at 1000
+  // and the masks the launch was bound by its waves, in FP32 too: 232 -> 181 us in FP32 at 1000
   // cameras with 200 000 points, 44 -> 33 us in FP64 at 137 cameras with 9001; in FP64 at 1000
-  // cameras it stays at 240 us, bound by the copies' traffic.
+  // cameras 243 -> 230 us, bound by the copies' traffic.
   int ix[NI];
   fetch_idx(q_begin, ix);
   int q = q_begin;
@@ -587,6 +593,8 @@ __global__ void __launch_bounds__(256) rcs_assemble_kernel(
     consume.template operator()<true>(q, lds_z[w]);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last index loads
+#pragma unroll
+  for (int u = 0; u < NI; ++u) asm volatile("" ::"v"(ix[u]));  // .. whose values are used on any path
   const d4 sum = acc;
   const int j = row;
   if (j >= ND) return;
