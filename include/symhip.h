@@ -400,7 +400,10 @@ int symhip_cholesky_factorize(symhip_cholesky_t c, const double* values);
    factor is then FP32-accurate in the updates; Solve does not refine (the optimizer's
    SYMHIP_PRECISION_F32_UPDATES form does). Call before the first Factorize. */
 int symhip_cholesky_set_f32_updates(symhip_cholesky_t c, int32_t on);
-/* Solve(b) for nrhs column-major right-hand sides (host buffers). */
+/* Solve(b) for nrhs column-major right-hand sides (host buffers). With more than one, the handle
+   keeps a workspace of five device vectors per right-hand side until it is destroyed: at most 256 MB
+   (or four right-hand sides where these take more), further ones go in several passes, and where the
+   device has no room for it fewer go at a time. */
 int symhip_cholesky_solve(symhip_cholesky_t c, const double* b, double* x, int32_t nrhs);
 /* inv_permutation (new -> old), the reference's Permutation().inverse() convention. */
 int symhip_cholesky_permutation(symhip_cholesky_t c, int32_t* inv_perm);

@@ -512,25 +512,17 @@ int symhip_cholesky_solve(symhip_cholesky_t c, const double* b, double* x, int32
   return guarded([&] {
     ensure_cholesky_device(c);
     const int32_t n = c->sym.n;
-    // several right-hand sides go through the solver together, as many as its workspace takes
-    // (fewer, down to one at a time, where the device has no room for it)
+    // Several right-hand sides go through the solver together, as many as its workspace takes
+    // (fewer, down to one at a time, where the device has no room for it). Together is the faster
+    // way from two on at every size: two 162 us against 213 one after the other at 1501 poses, 420
+    // against 520 at 10 000, 1.84 ms against 2.06 at 100 000; four 184 against 425 us at 1501.
     int32_t per = nrhs > 1 && n > 0 ? c->ldlt.many_capacity(nrhs) : 1;
-    auto room = [&](int32_t m) {
+    per = symhip::reserve_at_most(per, [&](int32_t m) {
       const size_t need = (size_t)std::max(1, n) * m;
       if (c->b.size() < need) c->b.resize(need);
       if (c->x.size() < need) c->x.resize(need);
       if (m > 1) c->ldlt.reserve_many(m, c->stream);
-    };
-    for (;;) {
-      try {
-        room(per);
-        break;
-      } catch (const symhip::Error&) {
-        if (per == 1) throw;
-        (void)hipGetLastError();
-        per /= 2;
-      }
-    }
+    });
     for (int32_t k = 0; k < nrhs; k += per) {
       const int32_t m = std::min(per, nrhs - k);
       const size_t len = (size_t)n * m;

@@ -4,17 +4,13 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
-#include <stdexcept>
 #include <string>
 #include <vector>
 
 #include "../../include/symhip_types.h"
+#include "./error.h"
 
 namespace symhip {
-
-struct Error : std::runtime_error {
-  using std::runtime_error::runtime_error;
-};
 
 #define SYMHIP_CHECK(cond, msg)                                  \
   do {                                                           \
@@ -55,7 +51,16 @@ class DBuf {
   void resize(size_t n) {
     if (n == n_) return;
     release();
-    if (n) HIP_OK(hipMalloc(&p_, n * sizeof(T)));
+    if (n) {
+      const hipError_t e = hipMalloc(&p_, n * sizeof(T));
+      if (e != hipSuccess) p_ = nullptr;
+      if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();  // reported here, not by the next launch's check
+        throw OutOfMemory("symhip: out of device memory allocating " +
+                          std::to_string(n * sizeof(T)) + " bytes");
+      }
+      HIP_OK(e);
+    }
     n_ = n;
   }
   void release() {
