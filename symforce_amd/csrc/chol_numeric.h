@@ -92,8 +92,9 @@ class SupernodalLDLT {
   DBuf<int32_t> counter_;  // per-supernode arrival counters of the backward pass (self-resetting)
   DBuf<double> many_y_, many_yout_, many_part_;  // solve_many
   DBuf<int32_t> many_counter_;                   // per (right-hand-side group, supernode)
-  DBuf<int64_t> scat_col_;
-  DBuf<int32_t> panel_src_, diag_pos_;  // factorize(): what each panel entry is assembled from
+  DBuf<int64_t> asm_map_, scat_col_;
+  int64_t nnz_ = 0;
+  DBuf<int32_t> panel_src_, diag_pos_;  // small panels: what each entry is assembled from
   DBuf<int32_t> rows_, perm_, upd_rel_, scat_rel_;
   DBuf<uint8_t> trsm_tasks_, upd_tasks_, solve_tasks_, chain_tasks_;  // per-level task lists (chol_numeric.hip)
   // work lists (flattened over levels)

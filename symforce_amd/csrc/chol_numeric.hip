@@ -42,36 +42,40 @@ struct SnTask {
   int32_t s, a, b, pad;  // supernode; chunk or tile row; tile column
 };
 
-// What a panel entry is assembled from (src): q >= 0 is entry q of the matrix, -2 - j its diagonal
-// entry of column j (at diag[j], -1 where the matrix has none), kPanelFill neither (fill-in, zero).
-// Built on the device from the matrix's map: the list is as long as the panels, and written and
-// uploaded by the host it took a 100 000-node pose graph's set-up from 175 to 195 ms.
+// Assembly of A + diag(damping) (damping null: of A) into the panels. The matrix's map holds the
+// panel place of every entry off the diagonal, ~j for column j's diagonal entry, which takes the
+// damping, and behind the nnz entries the diagonal's places by column.
+//
+// Panels of up to kListPanel entries: by a list of what each panel entry is assembled from (src,
+// built on the device: q >= 0 is entry q of the matrix, -2 - j the diagonal entry of column j, at
+// diag[j], kPanelFill neither), every entry written once, in one launch. Larger ones: zeroed, then
+// the matrix scattered into them. The list is read for every panel entry, four fifths of them
+// fill-in, and its dependent loads keep it at 2.9 TB/s; the second launch costs ~3 us. From
+// assembly to factorization on pose graphs, list against scatter: panels of 0.85 M entries 7.6
+// against 11.0 us, 3.3 M 16.4 / 19.5, 6.6 M 26.9 / 26.7, 13.3 M 51.8 / 37.0, 33 M (100 000 nodes)
+// 137 / 94 (of which 44 zero 266 MB), where the list also held 133 MB against the map's 50.
+constexpr int64_t kListPanel = 6 << 20;
 constexpr int32_t kPanelFill = -1;
 __global__ void panel_fill_kernel(int64_t size, int32_t* __restrict__ src) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < size;
        i += (int64_t)gridDim.x * blockDim.x)
     src[i] = kPanelFill;
 }
-__global__ void panel_entries_kernel(int64_t nnz, const int64_t* __restrict__ map,
-                                     int32_t* __restrict__ src) {
-  const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (q < nnz) src[map[q]] = (int32_t)q;
-}
-__global__ void panel_diagonal_kernel(int32_t n, const int32_t* __restrict__ diag,
-                                      const int64_t* __restrict__ map, int32_t* __restrict__ src) {
-  const int32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < n && diag[j] >= 0) src[map[diag[j]]] = -2 - j;
+__global__ void panel_list_kernel(int64_t nnz, const int64_t* __restrict__ map,
+                                  int32_t* __restrict__ src) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= nnz) return;
+  const int64_t p = map[i];
+  if (p >= 0) src[p] = (int32_t)i;
+  else src[map[nnz + ~p]] = (int32_t)(-2 - ~p);
 }
 
-// The panels of A + diag(damping) (damping null: of A), every entry written once: bound by the
-// panel's 12 bytes per entry. Zeroing the panels and scattering the matrix into them took two
-// launches and wrote its lines twice.
-__global__ void __launch_bounds__(256) assemble_kernel(int64_t size,
-                                                       const int32_t* __restrict__ src,
-                                                       const int32_t* __restrict__ diag,
-                                                       const double* __restrict__ vals,
-                                                       const double* __restrict__ damping,
-                                                       double* __restrict__ panel) {
+__global__ void __launch_bounds__(256) assemble_list_kernel(int64_t size,
+                                                            const int32_t* __restrict__ src,
+                                                            const int32_t* __restrict__ diag,
+                                                            const double* __restrict__ vals,
+                                                            const double* __restrict__ damping,
+                                                            double* __restrict__ panel) {
   const int64_t i = 2 * (blockIdx.x * (int64_t)256 + threadIdx.x);
   if (i >= size) return;
   auto value = [&](int32_t c) __attribute__((always_inline)) {
@@ -86,6 +90,22 @@ __global__ void __launch_bounds__(256) assemble_kernel(int64_t size,
     *reinterpret_cast<double2*>(panel + i) = make_double2(value(c.x), value(c.y));
   } else {
     panel[i] = value(src[i]);
+  }
+}
+
+__global__ void __launch_bounds__(256) assemble_scatter_kernel(int64_t nnz,
+                                                               const int64_t* __restrict__ map,
+                                                               const double* __restrict__ vals,
+                                                               const double* __restrict__ damping,
+                                                               double* __restrict__ panel) {
+  for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < nnz; i += (int64_t)gridDim.x * 256) {
+    int64_t p = map[i];
+    double v = vals[i];
+    if (p < 0) {
+      if (damping) v += damping[~p];
+      p = map[nnz + ~p];
+    }
+    panel[p] = v;
   }
 }
 
@@ -1071,28 +1091,33 @@ void SupernodalLDLT::setup(const CholSymbolic& sym, const int32_t* colptr, const
   SYMHIP_CHECK(sym.max_snode_cols <= kMaxCols, "supernode wider than the kernel tile");
   sym_ = sym;
   panel_.resize(std::max<int64_t>(1, sym.panel_size()));
-  DBuf<int64_t> map_dev;
   std::vector<int64_t> map;
   std::vector<int32_t> diag;
+  nnz_ = 0;
   if (colptr) {
     map = chol_assembly_map(sym, colptr, rowind);
-    diag.assign(std::max(1, sym.n), -1);
+    diag.assign(std::max(1, sym.n), 0);
+    nnz_ = (int64_t)map.size();
+    map.resize(std::max<int64_t>(1, nnz_ + sym.n), -1);
     for (int32_t j = 0; j < sym.n; ++j)
       for (int32_t q = colptr[j]; q < colptr[j + 1]; ++q)
-        if (rowind[q] == j) diag[j] = q;
+        if (rowind[q] == j) {
+          diag[j] = q;
+          map[nnz_ + j] = map[q];
+          map[q] = ~(int64_t)j;
+        }
     diag_pos_.upload(diag, s);
-    panel_src_.resize(panel_.size());
-    map_dev.upload(map, s);
-    const int64_t size = (int64_t)panel_.size(), nnz = (int64_t)map.size();
-    hipLaunchKernelGGL(panel_fill_kernel, dim3((int)std::min<int64_t>(grid_for(size, 256), 4096)),
-                       dim3(256), 0, s, size, panel_src_.get());
-    if (nnz) {
-      hipLaunchKernelGGL(panel_entries_kernel, dim3(grid_for(nnz, 256)), dim3(256), 0, s, nnz,
-                         map_dev.get(), panel_src_.get());
-      hipLaunchKernelGGL(panel_diagonal_kernel, dim3(grid_for(sym.n, 256)), dim3(256), 0, s, sym.n,
-                         diag_pos_.get(), map_dev.get(), panel_src_.get());
+    asm_map_.upload(map, s);
+    const int64_t size = sym.panel_size();
+    if (size > 0 && size <= kListPanel) {
+      panel_src_.resize(size);
+      hipLaunchKernelGGL(panel_fill_kernel, dim3(std::min(grid_for(size, 256), 4096)), dim3(256), 0,
+                         s, size, panel_src_.get());
+      if (nnz_)
+        hipLaunchKernelGGL(panel_list_kernel, dim3(grid_for(nnz_, 256)), dim3(256), 0, s, nnz_,
+                           asm_map_.get(), panel_src_.get());
+      HIP_OK(hipGetLastError());
     }
-    HIP_OK(hipGetLastError());
   }
   D_.resize(std::max(1, sym.n));
   y_.resize(std::max(1, sym.n));
@@ -1219,8 +1244,15 @@ void SupernodalLDLT::factorize(const double* a_values, hipStream_t s, const doub
   fused_ = b != nullptr;
   HIP_OK(hipGraphLaunch(cached_graph(fact_graphs_, {a_values, damping, b}, nullptr, 1.0, s, [&] {
     const int64_t size = sym_.panel_size();
-    hipLaunchKernelGGL(assemble_kernel, dim3(grid_for(size, 512)), dim3(256), 0, s, size,
-                       panel_src_.get(), diag_pos_.get(), a_values, damping, panel_.get());
+    if (panel_src_.size()) {
+      hipLaunchKernelGGL(assemble_list_kernel, dim3(grid_for(size, 512)), dim3(256), 0, s, size,
+                         panel_src_.get(), diag_pos_.get(), a_values, damping, panel_.get());
+    } else {
+      fill_zero(panel_.get(), size, s);
+      if (nnz_)
+        hipLaunchKernelGGL(assemble_scatter_kernel, dim3(std::min(grid_for(nnz_, 256), 8192)),
+                           dim3(256), 0, s, nnz_, asm_map_.get(), a_values, damping, panel_.get());
+    }
     launch_factorize(b, s);
   }), s));
 }

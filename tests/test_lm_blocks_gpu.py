@@ -2,7 +2,7 @@
 one block into another while the constants reach a block with its first use in a run, so a second
 run of one optimizer with other constants, runs with rejected steps (which change the blocks' order)
 and residual / state counts around the 256-thread blocks of the reductions are held to the oracle.
-Also the damped assembly at the odd panel sizes of its paired stores."""
+Also the damped assembly at the odd panel sizes of its paired stores, and its two ways."""
 import numpy as np
 import pytest
 
@@ -66,3 +66,23 @@ def test_assembly_of_odd_panels(n):
         want = np.linalg.solve(full, b)
         # diagonally dominant: condition below (5 + 2) / (4 - 2); both solutions backward stable
         assert np.abs(chol.solve(b) - want).max() <= 4 * n * EPS * 3.5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("damping", [dict(), dict(use_diagonal_damping=1)])
+def test_assembly_by_list_and_by_scatter(damping):
+    """Panels below and above the size from which the matrix is scattered into zeroed panels: one
+    pose graph in two elimination orders, whose panels lie on either side, and the larger one
+    twice on one optimizer (every panel entry is written again)."""
+    prob = capi.gen_pose_graph(18500, 5550, 42)
+    params = capi.default_params(iterations=4, early_exit_min_reduction=0.0, **damping)
+    runs = []
+    for ordering, small in ((capi.ORDERING_NESTED_DISSECTION, True),
+                            (capi.ORDERING_MIN_DEGREE, False)):
+        opt = capi.HipOptimizer(prob, params, capi.solver_options(ordering=ordering))
+        assert (opt.solver_info()["panel"] <= 6 << 20) == small
+        runs.append(opt.optimize())
+    runs.append(opt.optimize(prob.values))
+    for other in runs[1:]:
+        assert_same_trajectory(other, runs[0], rtol=1e-8)
+        np.testing.assert_allclose(other["values"], runs[0]["values"], rtol=0,
+                                   atol=1e-8 * np.abs(runs[0]["values"]).max())
