@@ -62,6 +62,9 @@ class SupernodalLDLT {
                      double* values, hipStream_t s) const;
 
  private:
+  // a vector's length in whole cache lines (32 entries: 128 bytes of the smallest type)
+  static size_t line_round(int32_t n) { return ((size_t)n + 31) / 32 * 32; }
+  int32_t* ticket() const { return counter_.get() + line_round(sym_.n_snodes); }
   void launch_factorize(const double* b, hipStream_t s);
   void launch_solve(const double* b, double* x, hipStream_t s);
   void launch_backward(double* x, double sign, hipStream_t s);
@@ -86,21 +89,23 @@ class SupernodalLDLT {
   bool fused_ = false;  // the last factorization ran the forward solve
   bool f32_updates_ = false;
   CholSymbolic sym_;
-  DBuf<double> panel_, l11_, D_, y_, yout_, part_;
-  DBuf<unsigned long long> ysol_;  // the backward launch's results as its blocks see them
-  DBuf<int32_t> ticket_;
-  DBuf<int32_t> counter_;  // per-supernode arrival counters of the backward pass (self-resetting)
+  DBuf<double> panel_, l11_;
+  DBuf<double> vectors_;  // D_, y_, yout_, part_ and ysol_ (one allocation: set-up pays for each)
+  double *D_ = nullptr, *y_ = nullptr, *yout_ = nullptr, *part_ = nullptr;
+  unsigned long long* ysol_ = nullptr;  // the backward launch's results as its blocks see them
+  // per-supernode arrival counters of the backward pass (self-resetting); its ticket on a line behind
+  DBuf<int32_t> counter_;
   DBuf<double> many_y_, many_yout_, many_part_;  // solve_many
   DBuf<int32_t> many_counter_;                   // per (right-hand-side group, supernode)
   DBuf<int64_t> asm_map_, scat_col_;
   int64_t nnz_ = 0;
   DBuf<int32_t> panel_src_, diag_pos_;  // small panels: what each entry is assembled from
   DBuf<int32_t> rows_, perm_, upd_rel_, scat_rel_;
-  DBuf<uint8_t> trsm_tasks_, upd_tasks_, solve_tasks_, chain_tasks_;  // per-level task lists (chol_numeric.hip)
+  DBuf<uint8_t> trsm_tasks_, upd_tasks_, solve_tasks_;  // per-level task lists (chol_numeric.hip)
   // work lists (flattened over levels)
   std::vector<int32_t> lvl_snode_ptr_, lvl_trsm_ptr_, lvl_upd_ptr_, lvl_solve_ptr_;
   DBuf<int32_t> lvl_snodes_;
-  int32_t chain_levels_ = 0, n_chain_ = 0;  // levels and tasks of the backward launch
+  int32_t chain_levels_ = 0, n_chain_ = 0;  // of the backward launch: levels, (the last) solve tasks
 };
 
 }  // namespace symhip

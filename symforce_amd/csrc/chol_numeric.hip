@@ -808,11 +808,12 @@ __device__ __forceinline__ double wait_value(const unsigned long long* p) {
 // system's 38 levels, now 3.1 (an optimizer run of ten solves 23.2 -> 21.6 ms; 137 cameras 5.94 ->
 // 5.35 ms; 2503-node pose graph 2.05 -> 1.89 ms).
 //
-// Every wait ends: a block's task is the ticket it draws when it starts, tasks are listed from the
-// root level down with chunk 0 last in each supernode, and a block waits only for tasks listed
-// before its own, whose blocks have therefore started; the earliest unfinished one waits for none.
+// Every wait ends: a block's task is the ticket it draws when it starts, counted back from the last
+// solve task (last): from the root level down and, a supernode's chunks being listed in their order,
+// with chunk 0 last in each supernode. A block waits only for tasks drawn before its own, whose
+// blocks have therefore started; the earliest unfinished one waits for none.
 __global__ void __launch_bounds__(256) bwd_chain_kernel(
-    const SnTask* __restrict__ tasks, const int32_t* __restrict__ rows,
+    const SnTask* __restrict__ last, const int32_t* __restrict__ rows,
     const double* __restrict__ panel, const double* __restrict__ l11, const double* __restrict__ D,
     double* __restrict__ yout, unsigned long long* ysol, double* part, int32_t* counter,
     int32_t* ticket) {
@@ -826,7 +827,7 @@ __global__ void __launch_bounds__(256) bwd_chain_kernel(
   __syncthreads();
   const int t = __builtin_amdgcn_readfirstlane(drawn);
   if (t >= (int)gridDim.x) return;  // uniform; not after a permute_kernel, which resets the ticket
-  const SnTask tk = tasks[t];
+  const SnTask tk = last[-t];
   const int s = tk.s, chunk = tk.a;
   const SnDesc sd = tk.d;
   const int n = sd.ncols, ld = sd.ld, mb = ld - n;
@@ -1096,20 +1097,15 @@ void SupernodalLDLT::setup(const CholSymbolic& sym, const int32_t* colptr, const
   nnz_ = 0;
   if (colptr) {
     map = chol_assembly_map(sym, colptr, rowind);
-    diag.assign(std::max(1, sym.n), 0);
-    nnz_ = (int64_t)map.size();
-    map.resize(std::max<int64_t>(1, nnz_ + sym.n), -1);
-    for (int32_t j = 0; j < sym.n; ++j)
-      for (int32_t q = colptr[j]; q < colptr[j + 1]; ++q)
-        if (rowind[q] == j) {
-          diag[j] = q;
-          map[nnz_ + j] = map[q];
-          map[q] = ~(int64_t)j;
-        }
-    diag_pos_.upload(diag, s);
+    nnz_ = colptr[sym.n];
     asm_map_.upload(map, s);
     const int64_t size = sym.panel_size();
     if (size > 0 && size <= kListPanel) {
+      diag.assign(sym.n, 0);
+      for (int32_t j = 0; j < sym.n; ++j)
+        for (int32_t q = colptr[j]; q < colptr[j + 1]; ++q)
+          if (rowind[q] == j) diag[j] = q;
+      diag_pos_.upload(diag, s);
       panel_src_.resize(size);
       hipLaunchKernelGGL(panel_fill_kernel, dim3(std::min(grid_for(size, 256), 4096)), dim3(256), 0,
                          s, size, panel_src_.get());
@@ -1119,13 +1115,14 @@ void SupernodalLDLT::setup(const CholSymbolic& sym, const int32_t* colptr, const
       HIP_OK(hipGetLastError());
     }
   }
-  D_.resize(std::max(1, sym.n));
-  y_.resize(std::max(1, sym.n));
-  yout_.resize(std::max(1, sym.n));
-  part_.resize(std::max(1, sym.n));
-  ysol_.resize(std::max(1, sym.n));
-  ticket_.resize(1);
-  counter_.resize(std::max(1, sym.n_snodes));
+  const size_t len = line_round(std::max(1, sym.n));
+  vectors_.resize(5 * len);
+  D_ = vectors_.get();
+  y_ = D_ + len;
+  yout_ = y_ + len;
+  part_ = yout_ + len;
+  ysol_ = reinterpret_cast<unsigned long long*>(part_ + len);
+  counter_.resize(line_round(sym.n_snodes) + 1);
   fill_zero_i32(counter_.get(), counter_.size(), s);
   rows_.upload(sym.sn_rows, s);
   perm_.upload(sym.perm, s);
@@ -1217,22 +1214,11 @@ void SupernodalLDLT::setup(const CholSymbolic& sym, const int32_t* colptr, const
   // Backward in one launch: the levels from the root down to the first with more blocks than are
   // resident (two to a CU). Below it a level's time is its blocks', not its chain's, and
   // bwd_kernel's lean form runs four to a CU.
-  std::vector<int32_t> chain;
-  chain_levels_ = 0;
-  for (int l = sym.n_levels - 1; l >= 0; --l, ++chain_levels_) {
+  for (chain_levels_ = 0; chain_levels_ < sym.n_levels; ++chain_levels_) {
+    const int l = sym.n_levels - 1 - chain_levels_;
     if (lvl_solve_ptr_[l + 1] - lvl_solve_ptr_[l] > 2 * kCus) break;
-    for (int q = lvl_solve_ptr_[l]; q < lvl_solve_ptr_[l + 1];) {
-      int e = q + 1;  // a supernode's chunks, the first one last
-      while (e < lvl_solve_ptr_[l + 1] && sol[2 * e] == sol[2 * q]) ++e;
-      for (int c = e - 1; c >= q; --c) {
-        chain.push_back(sol[2 * c]);
-        chain.push_back(sol[2 * c + 1]);
-      }
-      q = e;
-    }
   }
-  n_chain_ = (int32_t)chain.size() / 2;
-  upload_tasks(chain, 2, chain_tasks_);
+  n_chain_ = lvl_solve_ptr_[sym.n_levels] - lvl_solve_ptr_[sym.n_levels - chain_levels_];
   upload_tasks(dt, 2, trsm_tasks_);
   upload_tasks(upd, 3, upd_tasks_);
   HIP_OK(hipStreamSynchronize(s));
@@ -1327,7 +1313,7 @@ void SupernodalLDLT::solve_many(const double* b, double* x, int32_t nrhs, hipStr
     const int nb = lvl_solve_ptr_[l + 1] - lvl_solve_ptr_[l];
     hipLaunchKernelGGL(bwd_many_kernel, dim3(nb, groups), dim3(256), 0, s,
                        tasks + lvl_solve_ptr_[l], n, sym_.n_snodes, nrhs, rows_.get(),
-                       panel_.get(), l11_.get(), D_.get(), many_yout_.get(), many_part_.get(),
+                       panel_.get(), l11_.get(), D_, many_yout_.get(), many_part_.get(),
                        many_counter_.get());
   }
   hipLaunchKernelGGL(unpermute_many_kernel, pg, dim3(256), 0, s, n, nrhs, perm_.get(),
@@ -1361,24 +1347,24 @@ void SupernodalLDLT::launch_factorize(const double* b, hipStream_t s) {
   const SnTask* upd = reinterpret_cast<const SnTask*>(upd_tasks_.get());
   if (b)
     hipLaunchKernelGGL(permute_kernel, dim3(grid_for(sym_.n, 256)), dim3(256), 0, s, sym_.n,
-                       perm_.get(), b, y_.get(), part_.get(), ysol_.get(), ticket_.get());
+                       perm_.get(), b, y_, part_, ysol_, ticket());
   for (int l = 0; l < sym_.n_levels; ++l) {
     const int nt = lvl_trsm_ptr_[l + 1] - lvl_trsm_ptr_[l];
     if (nt) {
       if (b)
         hipLaunchKernelGGL(diag_trsm_kernel<true>, dim3(nt), dim3(kDiagThreads), 0, s,
                            trsm + lvl_trsm_ptr_[l], panel_.get(),
-                           l11_.get(), D_.get(), rows_.get(), y_.get(), yout_.get());
+                           l11_.get(), D_, rows_.get(), y_, yout_);
       else
         hipLaunchKernelGGL(diag_trsm_kernel<false>, dim3(nt), dim3(kDiagThreads), 0, s,
                            trsm + lvl_trsm_ptr_[l], panel_.get(),
-                           l11_.get(), D_.get(), nullptr, nullptr, nullptr);
+                           l11_.get(), D_, nullptr, nullptr, nullptr);
     }
     const int nu = lvl_upd_ptr_[l + 1] - lvl_upd_ptr_[l];
     if (nu) {
       auto kern = f32_updates_ ? update_kernel<kTile, float> : update_kernel<kTile, double>;
       hipLaunchKernelGGL(kern, dim3(nu), dim3(256), 0, s, upd + lvl_upd_ptr_[l], panel_.get(),
-                         D_.get(), scat_col_.get(), scat_rel_.get(), upd_rel_.get());
+                         D_, scat_col_.get(), scat_rel_.get(), upd_rel_.get());
     }
   }
   HIP_OK(hipGetLastError());
@@ -1388,12 +1374,12 @@ void SupernodalLDLT::launch_solve(const double* b, double* x, hipStream_t s) {
   const int n = sym_.n;
   const SnTask* tasks = reinterpret_cast<const SnTask*>(solve_tasks_.get());
   hipLaunchKernelGGL(permute_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, n, perm_.get(), b,
-                     y_.get(), part_.get(), ysol_.get(), ticket_.get());
+                     y_, part_, ysol_, ticket());
   for (int l = 0; l < sym_.n_levels; ++l) {
     const int nb = lvl_solve_ptr_[l + 1] - lvl_solve_ptr_[l];
     hipLaunchKernelGGL(fwd_kernel, dim3(nb), dim3(256), 0, s,
                        tasks + lvl_solve_ptr_[l], rows_.get(),
-                       panel_.get(), l11_.get(), y_.get(), yout_.get());
+                       panel_.get(), l11_.get(), y_, yout_);
   }
   launch_backward(x, 1.0, s);
 }
@@ -1405,18 +1391,16 @@ void SupernodalLDLT::launch_backward(double* x, double sign, hipStream_t s) {
   const SnTask* tasks = reinterpret_cast<const SnTask*>(solve_tasks_.get());
   if (n_chain_)
     hipLaunchKernelGGL(bwd_chain_kernel, dim3(n_chain_), dim3(256), 0, s,
-                       reinterpret_cast<const SnTask*>(chain_tasks_.get()), rows_.get(),
-                       panel_.get(), l11_.get(), D_.get(), yout_.get(), ysol_.get(), part_.get(),
-                       counter_.get(), ticket_.get());
+                       tasks + lvl_solve_ptr_[sym_.n_levels] - 1, rows_.get(), panel_.get(),
+                       l11_.get(), D_, yout_, ysol_, part_, counter_.get(), ticket());
   for (int l = sym_.n_levels - 1 - chain_levels_; l >= 0; --l) {
     const int nb = lvl_solve_ptr_[l + 1] - lvl_solve_ptr_[l];
     auto kern = nb > 2 * kCus ? bwd_kernel<true> : bwd_kernel<false>;
     hipLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, s, tasks + lvl_solve_ptr_[l], rows_.get(),
-                       panel_.get(), l11_.get(), D_.get(), yout_.get(), part_.get(),
-                       counter_.get());
+                       panel_.get(), l11_.get(), D_, yout_, part_, counter_.get());
   }
-  hipLaunchKernelGGL(unpermute_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, n, perm_.get(),
-                     yout_.get(), sign, x);
+  hipLaunchKernelGGL(unpermute_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, n, perm_.get(), yout_,
+                     sign, x);
   HIP_OK(hipGetLastError());
 }
 
@@ -1455,7 +1439,8 @@ void SupernodalLDLT::download_factor(std::vector<double>& panels, std::vector<do
   panels.resize(sym_.panel_size());
   d.resize(sym_.n);
   panel_.download(panels.data(), panels.size(), s);
-  D_.download(d.data(), d.size(), s);
+  if (!d.empty())
+    HIP_OK(hipMemcpyAsync(d.data(), D_, d.size() * sizeof(double), hipMemcpyDeviceToHost, s));
   HIP_OK(hipStreamSynchronize(s));
 }
 

@@ -504,25 +504,43 @@ std::vector<int64_t> chol_assembly_map(const CholSymbolic& s, const int32_t* col
   std::vector<int32_t> sn_of_col(n);
   for (int32_t k = 0; k < s.n_snodes; ++k)
     for (int32_t c = s.sn_col_begin[k]; c < s.sn_col_begin[k + 1]; ++c) sn_of_col[c] = k;
-  std::vector<int64_t> map(colptr[n]);
+  const int64_t nnz = colptr[n];
+  std::vector<int64_t> map(std::max<int64_t>(1, nnz + n), -1);
+  // the last row found below a supernode's own columns: a column's next entry is mostly in the same
+  // supernode and in that row (the entry's column moved on) or the one after it
+  int32_t last_t = -1, last_rp = 0;
   for (int32_t c = 0; c < n; ++c)
     for (int32_t q = colptr[c]; q < colptr[c + 1]; ++q) {
       int32_t pr = s.perm[rowind[q]], pc = s.perm[c];
       if (pr < pc) std::swap(pr, pc);  // lower triangle of the permuted matrix
       const int32_t t = sn_of_col[pc];
       const int32_t c0 = s.sn_col_begin[t], c1 = s.sn_col_begin[t + 1];
+      const int32_t* rows = s.sn_rows.data() + s.sn_rows_ptr[t];
+      const int32_t ld = s.sn_rows_ptr[t + 1] - s.sn_rows_ptr[t];
       int32_t rp;
       if (pr < c1) {
         rp = pr - c0;
       } else {
-        const int32_t* b = s.sn_rows.data() + s.sn_rows_ptr[t] + (c1 - c0);
-        const int32_t* e = s.sn_rows.data() + s.sn_rows_ptr[t + 1];
-        const int32_t* it = std::lower_bound(b, e, pr);
-        SYMHIP_CHECK(it != e && *it == pr, "internal: matrix entry outside the factor pattern");
-        rp = (int32_t)(it - (s.sn_rows.data() + s.sn_rows_ptr[t]));
+        if (t == last_t && rows[last_rp] == pr) {
+          rp = last_rp;
+        } else if (t == last_t && last_rp + 1 < ld && rows[last_rp + 1] == pr) {
+          rp = last_rp + 1;
+        } else {
+          const int32_t* it = std::lower_bound(rows + (c1 - c0), rows + ld, pr);
+          SYMHIP_CHECK(it != rows + ld && *it == pr,
+                       "internal: matrix entry outside the factor pattern");
+          rp = (int32_t)(it - rows);
+        }
+        last_t = t;
+        last_rp = rp;
       }
-      const int64_t ld = s.sn_rows_ptr[t + 1] - s.sn_rows_ptr[t];
-      map[q] = s.sn_panel_off[t] + (int64_t)(pc - c0) * ld + rp;
+      const int64_t place = s.sn_panel_off[t] + (int64_t)(pc - c0) * ld + rp;
+      if (rowind[q] == c) {
+        map[nnz + c] = place;
+        map[q] = ~(int64_t)c;
+      } else {
+        map[q] = place;
+      }
     }
   return map;
 }

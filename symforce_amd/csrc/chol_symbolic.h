@@ -74,7 +74,8 @@ void chol_symbolic(int32_t n, const int32_t* colptr, const int32_t* rowind,
                    const std::vector<int32_t>* given_node_order, int32_t max_cols,
                    CholSymbolic& out);
 
-// For each lower-pattern entry q of the input matrix, its position in the panel storage.
+// For each lower-pattern entry q of the input matrix off the diagonal, its position in the panel
+// storage; ~j for column j's diagonal entry, whose position is at [nnz + j] (-1 without one).
 std::vector<int64_t> chol_assembly_map(const CholSymbolic& s, const int32_t* colptr,
                                        const int32_t* rowind);
 
