@@ -202,7 +202,7 @@ class DeviceOptimizer {
   hipStream_t stream_ = nullptr;
   std::unique_ptr<SystemBackend> backend_;
   DBuf<double> values_[3];
-  DBuf<double> update_, last_update_, partials_, bold_partials_;
+  DBuf<double> update_, last_update_, partials_;
   DBuf<int32_t> retract_type_, retract_soff_, retract_toff_;
   LmDevState* dstate_ = nullptr;  // device
   LmDevState* hstate_ = nullptr;  // pinned host mirror, written by the finishing kernels

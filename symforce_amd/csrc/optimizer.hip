@@ -680,7 +680,7 @@ DeviceOptimizer::DeviceOptimizer(const symhip_problem_desc* d, const symhip_opti
   for (auto& v : values_) v.resize(std::max<int64_t>(1, host_.storage_total));
   update_.resize(std::max(1, host_.N));
   last_update_.resize(std::max(1, host_.N));
-  partials_.resize(4 * kReduceBlocks);
+  partials_.resize(5 * kReduceBlocks);  // lm_partials_kernel's four sums, the bold update's products
   std::vector<int32_t> rt, rs, rto;
   for (int32_t k : host_.state_keys) {
     rt.push_back(host_.types[k]);
@@ -1141,8 +1141,7 @@ bool DeviceOptimizer::iterate(std::vector<symhip_iteration_stats>& iters, int32_
                      backend_->rhs(init_), backend_->damping(), backend_->undamped_diagonal(),
                      epsilon_, (int64_t)N, nl, partials_.get());
   if (p_.enable_bold_updates && have_last_update_) {
-    bold_partials_.resize(kReduceBlocks);
-    double* part = bold_partials_.get();
+    double* part = partials_.get() + 4 * kReduceBlocks;
     dot(last_update_.get(), last_update_.get(), N, part, &dstate_->nl2, stream_);
     dot(update_.get(), update_.get(), N, part, &dstate_->nu2, stream_);
     dot(last_update_.get(), update_.get(), N, part, &dstate_->dotlu, stream_);
