@@ -14,6 +14,7 @@
 #include "./batch.h"
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <mutex>
 #include <type_traits>
@@ -480,7 +481,8 @@ batch_lm_kernel(BatchView v, symhip_optimizer_params p, double eps) {
         }
         if (p.use_unit_damping) d += lambda;
         damp[k] = d;
-        own[tri(k, k)] = dk + d;
+        // an infinite damping leaves no step; its reciprocal in the elimination would be a NaN
+        own[tri(k, k)] = fmin(dk + d, DBL_MAX);
       }
     }
     if (p.use_diagonal_damping && p.keep_max_diagonal_damping) have_max = true;

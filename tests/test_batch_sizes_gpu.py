@@ -63,3 +63,22 @@ def test_pose_without_matches():
             if prob.ftypes[f] == capi.FACTOR_MATCHING and poses[f] == first}
     assert drop
     check([without(prob, drop)], capi.default_params(iterations=15))
+
+
+@pytest.mark.parametrize("poses", [1, 2, 9, 33])
+@pytest.mark.parametrize("damping", [dict(), dict(use_diagonal_damping=1, use_unit_damping=0)])
+def test_infinite_damping(poses, damping):
+    """lambda = inf: a step of exact zeros, at whose unchanged error the run ends (lambda has no
+    bound to grow to); the oracle's linear error is inf * 0 and not compared."""
+    prob = capi.gen_localization(poses, 20, 0.5, seed=poses)
+    params = capi.default_params(iterations=5, initial_lambda=np.inf, lambda_upper_bound=np.inf,
+                                 **damping)
+    got = capi.HipBatch([prob], params).solve()["problems"][0]
+    ora = ow.OracleProblem(prob).optimize(params)
+    for k in ("status", "failure_reason", "best_index"):
+        assert got[k] == ora[k], k
+    assert [it["update_accepted"] for it in got["iterations"]] == \
+        [it["update_accepted"] for it in ora["iterations"]]
+    np.testing.assert_allclose([it["new_error"] for it in got["iterations"]],
+                               [it["new_error"] for it in ora["iterations"]], rtol=1e-12)
+    np.testing.assert_array_equal(got["values"], prob.values)
