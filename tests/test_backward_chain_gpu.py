@@ -1,5 +1,5 @@
 """The backward substitution's single launch over the narrow levels: supernodes of one and several
-128-row chunks, a wide level below the narrow ones, repeated solves on one handle, and right-hand
+128-row chunks, a wide level below the narrow ones and a narrow one below that, repeated solves on one handle, and right-hand
 sides that are not finite (results wait for one another by value, so every NaN has to arrive)."""
 import numpy as np
 import pytest
@@ -50,6 +50,30 @@ def test_wide_level_below(leaves, border):
     cols = np.repeat(np.arange(n), np.diff(cp))[keep]
     cp = np.searchsorted(cols, np.arange(n + 1)).astype(np.int32)
     chol = capi.HipCholesky(n, cp, ri[keep], ordering=capi.ORDERING_NATURAL)
+    chol.factorize(v[keep])
+    check(chol, a, 1)
+    check(chol, a, 2)
+
+
+@pytest.mark.parametrize("leaves,middle,border", [(2, 200, 260), (1, 180, 300), (2, 255, 257)])
+def test_narrow_level_below_a_wide_one(leaves, middle, border):
+    # `leaves` columns coupled to each middle column (one block each, 180 to 510 in all), the middle
+    # columns coupled to the border (three chunks each: more than 512 blocks), a dense border
+    n0, n1 = leaves * middle, (leaves + 1) * middle
+    n = n1 + border
+    rng = np.random.default_rng(n)
+    a = np.zeros((n, n))
+    a[n0 + np.arange(n0) // leaves, np.arange(n0)] = rng.uniform(-1, 1, n0)
+    a[n1:, n0:n1] = rng.standard_normal((border, middle)) / np.sqrt(n)
+    a = a + a.T
+    a[n1:, n1:] = spd(border, border)
+    a += 4 * np.eye(n)
+    _, cp, ri, v = dense_to_lower_csc(a)
+    keep = v != 0
+    cols = np.repeat(np.arange(n), np.diff(cp))[keep]
+    cp = np.searchsorted(cols, np.arange(n + 1)).astype(np.int32)
+    chol = capi.HipCholesky(n, cp, ri[keep], ordering=capi.ORDERING_NATURAL)
+    assert chol.info()["levels"] == 2 + -(-border // 64)
     chol.factorize(v[keep])
     check(chol, a, 1)
     check(chol, a, 2)

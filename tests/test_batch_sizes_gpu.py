@@ -2,7 +2,8 @@
 its middle pose (odd and even lengths, one and two poses have no or one eliminated pose), a pose's
 matching factors are dealt to 1, 2 or 4 lanes (more than 32, 17 to 32, up to 16 poses), and a pose
 may have no matching factor or no odometry to the next. Held to the oracle's trajectory with
-test_batch_gpu.py's tolerance."""
+test_batch_gpu.py's tolerance; the FP32-Jacobian form, whose steps are its own, to the oracle's
+minimum."""
 import numpy as np
 import pytest
 
@@ -37,6 +38,19 @@ def check(probs, params):
 def test_chain_lengths(poses):
     probs = [capi.gen_localization(poses, lm, 0.3, seed=10 * poses + lm) for lm in (9, 21, 40)]
     check(probs, capi.default_params(iterations=20))
+
+
+@pytest.mark.parametrize("poses", [1, 2, 16, 17, 32, 33, 64])
+def test_chain_lengths_fp32(poses):
+    probs = [capi.gen_localization(poses, lm, 0.3, seed=10 * poses + lm) for lm in (9, 21, 40)]
+    params = capi.default_params(iterations=40, early_exit_min_reduction=0.0)
+    res = capi.HipBatch(probs, params, precision=capi.PRECISION_F32_JAC).solve()["problems"]
+    for prob, got in zip(probs, res):
+        ora = ow.OracleProblem(prob).optimize(params)
+        assert got["iterations"][0]["new_error"] == \
+            pytest.approx(ora["iterations"][0]["new_error"], rel=1e-8)  # FP64 residuals
+        best, want = (r["iterations"][r["best_index"]]["new_error"] for r in (got, ora))
+        assert best == pytest.approx(want, rel=1e-8)
 
 
 @pytest.mark.parametrize("poses", [2, 7, 16, 33])

@@ -1,7 +1,8 @@
 """The LM run's three Values blocks and its fused reductions: the optimized keys are retracted from
 one block into another while the constants reach a block with its first use in a run, so a second
 run of one optimizer with other constants, runs with rejected steps (which change the blocks' order)
-and residual / state counts around the 256-thread blocks of the reductions are held to the oracle.
+and with bold updates (an accepted step that is not the best is what brings the third block in), and
+residual / state counts around the 256-thread blocks of the reductions are held to the oracle.
 Also the damped assembly at the odd panel sizes of its paired stores, and its two ways."""
 import numpy as np
 import pytest
@@ -42,6 +43,49 @@ def test_second_run_uses_its_own_constants(poses, lm, initial_lambda):
         assert_same_trajectory(got, ora, rtol=1e-8)
         np.testing.assert_allclose(got["values"], ora["values"], rtol=0,
                                    atol=1e-8 * max(1.0, np.abs(ora["values"]).max()))
+
+
+def moved_pixels(p, seed):
+    """The pixel measurements of a bundle adjustment (constants), moved by a pixel or so."""
+    rng = np.random.default_rng(seed)
+    v = p.values.copy()
+    for o, t in zip(p.storage_offsets, p.types):
+        if t == capi.TYPE_VECTOR2:
+            v[o:o + 2] += rng.standard_normal(2)
+    assert not np.array_equal(v, p.values)
+    return v
+
+
+def steps(run):
+    """A letter per step: r(ejected), a(ccepted), B(old: accepted without reducing the error)."""
+    return "".join("r" if not it["update_accepted"] else "a" if it["relative_reduction"] > 0 else "B"
+                   for it in run["iterations"] if it["iteration"] >= 0)
+
+
+@pytest.mark.parametrize("solver", [capi.SOLVER_CHOLESKY, capi.SOLVER_SCHUR])
+@pytest.mark.parametrize("cams,lam", [(4, capi.LAMBDA_STATIC), (4, capi.LAMBDA_DYNAMIC),
+                                      (8, capi.LAMBDA_STATIC)])
+def test_second_run_with_rejected_steps(cams, lam, solver):
+    prob = capi.gen_ba_circle(cams, 8 * cams, seed=cams)
+    params = capi.default_params(iterations=12, lambda_update_type=lam)
+    opt = capi.HipOptimizer(prob, params, capi.solver_options(linear_solver=solver))
+    for values in (prob.values, moved_pixels(prob, cams), prob.values):
+        ora = ow.OracleProblem(with_values(prob, values)).optimize(params)
+        assert "ra" in steps(ora), steps(ora)
+        assert_same_trajectory(opt.optimize(values=values), ora, rtol=1e-8)
+
+
+@pytest.mark.parametrize("solver", [capi.SOLVER_CHOLESKY, capi.SOLVER_SCHUR])
+def test_second_run_with_bold_updates(solver):
+    prob = capi.gen_ba_snavely(8, 160, 5)
+    params = capi.default_params(iterations=11, enable_bold_updates=1)
+    opt = capi.HipOptimizer(prob, params, capi.solver_options(linear_solver=solver))
+    for values in (prob.values, moved_pixels(prob, 8), prob.values):
+        ora = ow.OracleProblem(with_values(prob, values)).optimize(params)
+        assert "B" in steps(ora), steps(ora)
+        # A bold step is taken where the system is unstable: moving the oracle's start by 1e-13
+        # moves its records by up to 1e-9. (The other run's pixels move the first one by 3e-4.)
+        assert_same_trajectory(opt.optimize(values=values), ora, rtol=1e-7)
 
 
 @pytest.mark.parametrize("n", [1, 2, 3, 5, 16, 17, 23, 65])
