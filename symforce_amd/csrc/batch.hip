@@ -71,7 +71,8 @@ __device__ __forceinline__ int tri(int r, int c) { return r * (r + 1) / 2 + c; }
 // ratio and relative-reduction exit behave as in FP64 (FP32 residuals put a ~1e-7 floor under
 // the cost, which kept LM from its early exit on some problems). The products J^T J are formed
 // in FP64 from the FP32 Jacobians, so H stays positive semi-definite (FP32 sums of products
-// made a near-singular H slightly indefinite, and the block Cholesky then failed).
+// made a near-singular H slightly indefinite: the LDL^T takes no square roots and gives a finite
+// step there that need not descend, an iteration spent on its rejection).
 template <typename S>
 __device__ __forceinline__ double linearize(const BatchView& v, int b, int g0, int n, int lane) {
   double D[21] = {}, gv[6] = {}, Dn[21] = {}, gn[6] = {};

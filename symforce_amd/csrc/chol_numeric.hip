@@ -5,8 +5,9 @@
 //
 // The work per supernode is small (panels are at most 64 columns wide), so every kernel is
 // latency-bound: the kernels are written to avoid data-dependent branches (16 elimination steps
-// are unrolled over panels padded to 64 columns, the padding being an identity block) and chains of dependent global loads (each supernode's metadata is one descriptor,
-// scatter targets are precomputed per below-row).
+// are unrolled over panels padded to 64 columns, the padding being an identity block) and chains of
+// dependent global loads (each supernode's metadata is one descriptor, scatter targets are
+// precomputed per below-row).
 #include <algorithm>
 
 #include "./chol_numeric.h"

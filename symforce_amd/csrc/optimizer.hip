@@ -206,8 +206,8 @@ __global__ void factor_check_kernel(int32_t n, const int32_t* __restrict__ type,
   bad[f] = factor_finite_upto<1>(type[f], a) ? 0 : 1;
 }
 
-// Values::Retract over the optimized keys (opt/values.cc:314-327).
-// from the Init block into the New one, whose other keys hold their constants already.
+// Values::Retract over the optimized keys (opt/values.cc:314-327), from the Init block into the New
+// one, whose other keys hold their constants already.
 __global__ void retract_kernel(int32_t n, const int32_t* __restrict__ type,
                                const int32_t* __restrict__ soff, const int32_t* __restrict__ toff,
                                const double* __restrict__ update, const double* __restrict__ from,
@@ -360,10 +360,10 @@ __global__ void negate_kernel(int32_t n, const double* __restrict__ x, double* _
 }
 
 // out = b - A x (b non-null) or out = A x, for the symmetric A held as its lower CSC (colptr,
-// rowind, vals) plus the damping on its diagonal: row i of A is column i's entries (rows >= i) and the entries (i, j), j < i,
-// which tptr / tcol / tidx list per row (column j and the entry's index in vals). One thread
-// per row, FP64, no atomics: the residuals and products of the mixed-precision form's
-// refinement.
+// rowind, vals) plus the damping on its diagonal: row i of A is column i's entries (rows >= i) and
+// the entries (i, j), j < i, which tptr / tcol / tidx list per row (column j and the entry's index
+// in vals). One thread per row, FP64, no atomics: the residuals and products of the mixed-precision
+// form's refinement.
 __global__ void __launch_bounds__(256) sym_matvec_kernel(
     int32_t n, const int32_t* __restrict__ colptr, const int32_t* __restrict__ rowind,
     const double* __restrict__ vals, const int32_t* __restrict__ tptr,

@@ -399,9 +399,10 @@ __global__ void __launch_bounds__(256) point_elim_kernel(int32_t n_obs,
 // - sum_pairs Z_x Z_y^T. The pair sum is the product X Y^T with X = [Z_x1 Z_x2 ...] (ND x 3P)
 // and Y = [Z_y1 Z_y2 ...], so K = 3P is packed densely into FP64 matrix-core steps
 // (v_mfma_f64_16x16x4f64; a batch of eight pairs = 24 K entries = six MFMAs): at step h lane l
-// feeds A(i = l % 16, k = l / 16) = X(i, 4h + k) and B(k, j = l % 16) = Y(j, 4h + k) (rows
-// i >= ND and K entries past the block's pairs are zero) and holds D(l / 16 + 4 r, l % 16) in
-// accumulator register r (the FP64 16x16x4 output interleaves rows across the four lane groups).
+// feeds A(i = l % 16, k = l / 16) = X(i, 4h + k) and B(k, j = l % 16) = Y(j, 4h + k) (K entries
+// past the block's pairs are zero; rows i >= ND repeat row 0, their products are not stored) and
+// holds D(l / 16 + 4 r, l % 16) in accumulator register r (the FP64 16x16x4 output interleaves rows
+// across the four lane groups).
 // The pair list is padded so a batch reaching past the last block stays inside it. Diagonal
 // blocks carry no pairs: their sum_o Z_o Z_o^T (ZZ_a) comes from the per-camera reduction. Waves
 // take work items from a host-built list: (block, pair range, flags), blocks with many pairs
@@ -457,7 +458,7 @@ __global__ void __launch_bounds__(256) rcs_assemble_kernel(
   // in the MFMA layout touched ~10 lines per instruction for 288 useful bytes. Slot o of pair
   // p = o / 2 is its x (o even) or y (o odd), i.e. pairs[2 q + o]. At step h lane l reads its
   // operands from LDS: K = 4h + l / 16 is pair K / 3, column K % 3. Pairs past the item's end
-  // come from the next pairs or the padding (valid observations), masked by ok.
+  // come from the next pairs or the padding (valid observations) and are masked.
   constexpr int ZS = z_stride<ND, TW>(), NB = kRcsBatch, NH = NB * 3 / 4;
   constexpr int CPO = ZS * (int)sizeof(TW) / 16;
   constexpr int SLOTS = 2 * NB * CPO, NI = (SLOTS + 63) / 64;
