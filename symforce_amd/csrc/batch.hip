@@ -482,8 +482,10 @@ batch_lm_kernel(BatchView v, symhip_optimizer_params p, double eps) {
         }
         if (p.use_unit_damping) d += lambda;
         damp[k] = d;
-        // an infinite damping leaves no step; its reciprocal in the elimination would be a NaN
-        own[tri(k, k)] = fmin(dk + d, DBL_MAX);
+        // an infinite damping leaves no step; its reciprocal in the elimination would be a NaN (by
+        // fmin 499 problems take 153.4 us instead of 151.3)
+        const double h = dk + d;
+        own[tri(k, k)] = h == __builtin_huge_val() ? DBL_MAX : h;
       }
     }
     if (p.use_diagonal_damping && p.keep_max_diagonal_damping) have_max = true;
